@@ -82,6 +82,18 @@ uint64_t job_bytes(const gpi_job& j)
     return b * 21 / 20 + (1 << 20);
 }
 
+// Device bytes a 2-D forward run takes on top when they are there (the state and coefficients
+// of the several-step launches; without them the passes run).
+uint64_t job_optional_bytes(const gpi_job& j)
+{
+    const gpi_grid& g = j.grid;
+    if (g.ndim != 2) return 0;
+    const uint64_t h = (uint64_t)(g.order - 1), ld = (uint64_t)round_up(g.n[0] + (int64_t)h, 32);
+    const uint64_t slab = 4 * ld * ((uint64_t)g.n[2] + h);
+    const uint64_t face = std::max(ld, (uint64_t)g.n[2] + h), np = (uint64_t)std::max(g.npml, 0);
+    return (g.physics == 0 ? 5 * slab : 10 * slab) + (g.physics == 0 ? 4 : 8) * 2 * np * face * 4;
+}
+
 int run_job(gpi_ctx* c, const gpi_job& j)
 {
     uint64_t model = 0;
@@ -256,7 +268,7 @@ int gpi_jobs_submit(gpi_jobs* q, const gpi_job* job, uint64_t* ticket)
     Job x;
     x.ticket = q->next++;
     x.j = j;
-    x.est = est;
+    x.est = std::min(q->budget, est + job_optional_bytes(j));
     x.t_submit = now_ms();
     q->status[x.ticket] = 1;
     q->queue.push_back(x);

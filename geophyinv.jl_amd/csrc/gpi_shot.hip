@@ -4,6 +4,7 @@
 #include <map>
 
 #include "fdtd2d.h"
+#include "fdtd2d_steps.h"
 #include "fdtd3d.h"
 #include "gpi_util.h"
 #include "pass_extras.h"
@@ -48,6 +49,7 @@ int plan_sources(gpi_ctx* c, const Model& m, Scratch& S, int nsrc, const gpi_poi
     const int snb = d3 ? stress_blocks_3d(m, &sgx, &sgy) : stress_buckets_2d(m, &sgx);
     const int ty3 = d3 ? tile_rows_3d(m) : 1;
     out.pts.assign(nsrc, DevPoints{});
+    out.toff.assign(nsrc, {});
     std::vector<int> kinds(nsrc);
     bool vel_fused = true, str_fused = true;
     for (int q = 0; q < nsrc; ++q) {
@@ -138,6 +140,7 @@ int plan_sources(gpi_ctx* c, const Model& m, Scratch& S, int nsrc, const gpi_poi
         }
         D.ntarget = (int32_t)toff.size();
         toff.insert(toff.end(), roff.begin(), roff.end());
+        out.toff[q] = toff;
         int rc;
         if ((rc = S.put(&D.toff, toff)) || (rc = S.put(&D.tptr, tptr)) || (rc = S.put(&D.tsrc, tsrc)) ||
             (rc = S.put(&D.tw, tw)) || (rc = S.put(&D.blk, blk)))
@@ -502,15 +505,47 @@ int run_shot(gpi_ctx* c, Model& m, const gpi_shot* shot, Store* save)
     char* pack = nullptr;
     if (pack_bytes && (rc = S.alloc(&pack, pack_bytes))) return rc;
 
+    // several steps per launch where nothing is taken from the wavefield between the steps
+    StepPlan plan;
+    bool stepped = false;
+    if (g.ndim == 2 && !illum && !(save && !ckpt) && c->sample_ev.empty())
+        if ((rc = plan_steps_2d(c, m, S, nt, src, shot, rec, &plan, &stepped))) return rc;
+    // the launches of a shot end at checkpoints and snapshots
+    auto launch_steps = [&](int64_t it) {
+        int64_t n = std::min<int64_t>(plan.steps, nt - it);
+        if (ckpt) n = std::min(n, save->every - it % save->every);
+        for (int q = 0; q < shot->nsnap; ++q)
+            if (shot->snap_steps[q] >= it) n = std::min(n, shot->snap_steps[q] + 1 - it);
+        return (int)n;
+    };
+    if (stepped) {   // an even number of launches starts in the model's state, an odd one in the other
+        int64_t n = 0;
+        for (int64_t it = 0; it < nt; it += launch_steps(it)) ++n;
+        plan.cur = (int)(n & 1);
+    }
+
     // reset wavefields and CPML memory (reset_w2!, types.jl:101-113)
-    if ((rc = zero_state(c, m, st, c->stream))) return rc;
+    if ((rc = zero_state(c, m, stepped ? *plan.st[plan.cur] : st, c->stream))) return rc;
 
     // per step: velocity pass (records p at :177, sources of :202 ride along), then stress
     // pass (records v at :208, sources of :223 ride along), then boundary_save! (:229)
     Sampler smp(c, nt);
     int64_t launches = 0;
     HIPTRY(c, hipEventRecord(c->ev[0], c->stream));
-    for (int64_t it = 0; it < nt; ++it) {
+    for (int64_t it = 0; stepped && it < nt;) {
+        const int n = launch_steps(it);
+        run_steps_2d(m, plan, it, n, c->stream);
+        launches += plan.launches;
+        it += n;
+        const State& now = *plan.st[plan.cur];
+        if (ckpt && it % save->every == 0 && it / save->every <= (int64_t)save->ckpt.size())
+            if ((rc = copy_state(c, m, now, save->ckpt[it / save->every - 1], true, c->stream))) return rc;
+        for (int q = 0; q < shot->nsnap; ++q)
+            if (shot->snap_steps[q] == it - 1)
+                HIPTRY(c, hipMemcpyAsync(snap[q], now.field[shot->snap_field], sizeof(float) * (size_t)m.slab,
+                                         hipMemcpyDeviceToDevice, c->stream));
+    }
+    for (int64_t it = 0; !stepped && it < nt; ++it) {
         hipEvent_t* E = smp.at(it);
         XV.it = it;
         XS.it = it;

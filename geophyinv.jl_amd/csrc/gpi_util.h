@@ -72,6 +72,7 @@ struct Scratch;
 // pass keeps the reference's order of updates).  gpi_shot.hip.
 struct Sources {
     std::vector<DevPoints> pts;
+    std::vector<std::vector<int64_t>> toff;   // host copy of each set's toff
     std::vector<int> vfall, sfall;   // sets injected after the velocity / stress pass
 };
 // Forward sources kept by a checkpoint store: replayed, without receivers, when the
