@@ -175,6 +175,7 @@ int gpi_create(gpi_ctx** out, int device, uint64_t hbm_budget_bytes)
     size_t fr = 0, tot = 0;
     (void)hipMemGetInfo(&fr, &tot);
     c->budget = hbm_budget_bytes ? hbm_budget_bytes : (uint64_t)fr;
+    c->keep_cap = std::min<uint64_t>((uint64_t)tot / 32, (uint64_t)8 << 30);
     *out = c;
     return GPI_OK;
 }
@@ -186,6 +187,8 @@ void gpi_destroy(gpi_ctx* c)
     (void)hipStreamSynchronize(c->stream);
     for (Store* s : c->stores) free_store(c, s);
     for (Model* m : c->models) free_model(c, m);
+    trim_kept(c);
+    if (c->small.buf) (void)hipHostFree(c->small.buf);
     for (auto& e : c->ev) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->sample_ev) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(c->stream);
@@ -306,6 +309,7 @@ int gpi_model_free(gpi_ctx* c, uint64_t model)
     }
     c->models.erase(std::find(c->models.begin(), c->models.end(), m));
     free_model(c, m);
+    trim_kept(c);
     return GPI_OK;
 }
 

@@ -142,6 +142,14 @@ struct Ctx {
     hipEvent_t ev[4] = {};
     std::vector<hipEvent_t> sample_ev;   // 4 events per sampled step
     uint64_t budget = 0, used = 0;
+    // Buffers of finished calls kept for the next ones instead of hipFree (a hipMalloc and
+    // hipFree pair costs 0.1 ms for a small buffer and milliseconds for a segment of
+    // wavefields): at most keep_cap bytes, freed with a model or the context, or when memory
+    // or the budget runs short.  0: nothing is kept.
+    uint64_t keep_cap = 0, kept_bytes = 0;
+    std::multimap<size_t, void*> kept;                 // size -> block
+    std::unordered_map<void*, size_t> block_size;      // live and kept blocks that may be kept
+    PinnedStage small;                                 // ring for the small uploads of such a context
     std::string err;
     std::vector<Model*> models;
     std::vector<Store*> stores;

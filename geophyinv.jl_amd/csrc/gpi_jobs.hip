@@ -166,6 +166,7 @@ struct gpi_jobs {
     {
         gpi_ctx* c = nullptr;
         const int crc = gpi_create(&c, device, 0);
+        if (!crc) c->keep_cap = 0;   // the queue accounts for the running jobs' memory only
         for (;;) {
             Job job;
             {

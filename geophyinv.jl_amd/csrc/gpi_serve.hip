@@ -775,6 +775,7 @@ int gpi_server_create(int device, const gpi_server_opts* opts, gpi_server** out)
     if (v->o.chunk_steps == 0) v->o.chunk_steps = 32;
     int rc = gpi_create(&v->cc, device, 0);
     if (!rc) rc = gpi_create(&v->ac, device, 0);
+    if (!rc) v->cc->keep_cap = v->ac->keep_cap = 0;   // both have pools of their own
     if (rc) {
         if (v->cc) gpi_destroy(v->cc);
         delete v;

@@ -281,15 +281,15 @@ int alloc_store(gpi_ctx* c, Model& m, int64_t nt, Store** out)
             sd[ax] = 2 * NBOUND;
             s->strip_size[q][ax] = sd[0] * sd[1] * sd[2];
             int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&s->strip[q][ax],
-                               sizeof(float) * (size_t)(s->strip_size[q][ax] * nt));
+                               sizeof(float) * (size_t)(s->strip_size[q][ax] * nt), true);
             if (rc) return bail(rc);
         }
-        int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&s->snap[s->field[q]], sizeof(float) * (size_t)m.slab);
+        int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&s->snap[s->field[q]], sizeof(float) * (size_t)m.slab, true);
         if (rc) return bail(rc);
     }
     for (int f : {GPI_VX, GPI_VY, GPI_VZ}) {
         if (!field_codes(g.ndim, g.physics, f)) continue;
-        int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&s->snap[f], sizeof(float) * (size_t)m.slab);
+        int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&s->snap[f], sizeof(float) * (size_t)m.slab, true);
         if (rc) return bail(rc);
     }
     *out = s;
@@ -315,12 +315,12 @@ int alloc_checkpoint_store(gpi_ctx* c, Model& m, int64_t nt, int64_t every, Stor
     const size_t per = state_floats(m);
     s->ckpt.assign((size_t)std::max<int64_t>(K - 1, 0), nullptr);
     for (float*& p : s->ckpt) {
-        const int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&p, sizeof(float) * per);
+        const int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&p, sizeof(float) * per, true);
         if (rc) return bail(rc);
     }
     for (int f : {GPI_VX, GPI_VY, GPI_VZ}) {
         if (!field_codes(g.ndim, g.physics, f)) continue;
-        const int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&s->snap[f], sizeof(float) * (size_t)m.slab);
+        const int rc = dev_alloc(c, &s->allocs, &s->bytes, (void**)&s->snap[f], sizeof(float) * (size_t)m.slab, true);
         if (rc) return bail(rc);
     }
     *out = s;
@@ -709,7 +709,7 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
             free_allocs(c, st.allocs, st.bytes);
         }
     } h2{c, State{}};
-    int rc = alloc_state(c, m, &h2.st);
+    int rc = alloc_state(c, m, &h2.st, true);
     if (rc) return rc;
     const State& s2 = h2.st;
     PassExtras XV1{}, XS1{}, XV2{}, XS2{};
@@ -821,7 +821,7 @@ int gpi_adjoint_checkpoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi
             free_allocs(c, st.allocs, st.bytes);
         }
     } h2{c, State{}};
-    int rc = alloc_state(c, m, &h2.st);
+    int rc = alloc_state(c, m, &h2.st, true);
     if (rc) return rc;
     const State& s2 = h2.st;
     PassExtras XV2{}, XS2{};
@@ -977,7 +977,7 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
             free_allocs(c, st.allocs, st.bytes);
         }
     } h2{c, State{}};
-    int rc = alloc_state(c, m, &h2.st);
+    int rc = alloc_state(c, m, &h2.st, true);
     if (rc) return rc;
     const State& s2 = h2.st;
     PassExtras XV2{}, XS2{};
@@ -1157,7 +1157,7 @@ int gpi_born(gpi_ctx* c, uint64_t model, const gpi_shot* shot, const gpi_array* 
             free_allocs(c, st.allocs, st.bytes);
         }
     } h2{c, State{}};
-    if ((rc = alloc_state(c, m, &h2.st))) return rc;
+    if ((rc = alloc_state(c, m, &h2.st, true))) return rc;
     const State& w2 = h2.st;
     // coefficient perturbations on the device (absent ones are zero)
     const int ids[4] = {GPI_C_DTINVAVXIRHO, GPI_C_DTINVAVYIRHO, GPI_C_DTINVAVZIRHO, GPI_C_DTK};

@@ -41,7 +41,10 @@ inline bool is_velocity(int f) { return f == GPI_VX || f == GPI_VY || f == GPI_V
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 Model* find_model(gpi_ctx* c, uint64_t h);
-int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void** p, size_t bytes);
+// reuse: a buffer of one call, taken from and returned to the context's kept blocks
+int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void** p, size_t bytes,
+              bool reuse = false);
+void trim_kept(gpi_ctx* c);
 void free_allocs(gpi_ctx* c, std::vector<void*>& allocs, uint64_t& bytes);
 void free_model(gpi_ctx* c, Model* m);
 
@@ -50,7 +53,7 @@ void free_model(gpi_ctx* c, Model* m);
 int alloc_coef(gpi_ctx* c, Model& m, int id);
 
 // wavefields + CPML memory of one propagating wavefield of model m
-int alloc_state(gpi_ctx* c, const Model& m, State* st);
+int alloc_state(gpi_ctx* c, const Model& m, State* st, bool reuse = false);
 void free_state(gpi_ctx* c, State* st);
 int zero_state(gpi_ctx* c, const Model& m, const State& st, hipStream_t s);
 size_t psi_floats(const Model& m, int f);
@@ -140,7 +143,7 @@ struct Scratch {
     {
         void* q = nullptr;
         const size_t b = std::max<size_t>(sizeof(T) * count, 4);
-        int rc = c->arena ? arena_alloc(c, &q, b) : dev_alloc(c, &p, &bytes, &q, b);
+        int rc = c->arena ? arena_alloc(c, &q, b) : dev_alloc(c, &p, &bytes, &q, b, true);
         if (rc) return rc;
         *out = (T*)q;
         return GPI_OK;

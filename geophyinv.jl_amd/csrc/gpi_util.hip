@@ -112,11 +112,45 @@ Model* find_model(gpi_ctx* c, uint64_t h)
     return nullptr;
 }
 
-int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void** p, size_t bytes)
+void trim_kept(gpi_ctx* c)
+{
+    for (const auto& k : c->kept) {
+        c->block_size.erase(k.second);
+        (void)hipFree(k.second);
+    }
+    c->kept.clear();
+    c->kept_bytes = 0;
+}
+
+int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void** p, size_t bytes, bool reuse)
 {
     if (c->budget && c->used + bytes > c->budget)
         return fail(c, GPI_ENOMEM, "allocation of " + std::to_string(bytes) + " bytes exceeds the context's HBM budget");
-    hipError_t e = c->pool ? c->pool->alloc(p, bytes) : hipMalloc(p, bytes);
+    hipError_t e = hipSuccess;
+    if (c->pool) {
+        e = c->pool->alloc(p, bytes);
+    } else {
+        reuse = reuse && c->keep_cap;
+        *p = nullptr;
+        if (reuse) {
+            auto k = c->kept.lower_bound(bytes);
+            if (k != c->kept.end() && k->first <= bytes + bytes / 8 + 65536) {
+                *p = k->second;
+                c->kept_bytes -= k->first;
+                c->kept.erase(k);
+            }
+        }
+        if (!*p) {
+            if (c->kept_bytes && c->budget && c->used + c->kept_bytes + bytes > c->budget) trim_kept(c);
+            e = hipMalloc(p, bytes);
+            if (e != hipSuccess && c->kept_bytes) {
+                (void)hipGetLastError();
+                trim_kept(c);
+                e = hipMalloc(p, bytes);
+            }
+            if (e == hipSuccess && reuse) c->block_size[*p] = bytes;
+        }
+    }
     if (e != hipSuccess) return fail(c, GPI_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     c->used += bytes;
     owner->push_back(*p);
@@ -157,7 +191,17 @@ void free_allocs(gpi_ctx* c, std::vector<void*>& allocs, uint64_t& bytes)
     } else if (c->pool) {
         for (void* p : allocs) c->pool->free(p);
     } else {
-        for (void* p : allocs) (void)hipFree(p);
+        // the caller has drained the stream; a kept block is reused on the same stream only
+        for (void* p : allocs) {
+            auto b = c->block_size.find(p);
+            if (b != c->block_size.end() && c->kept_bytes + b->second <= c->keep_cap) {
+                c->kept.insert({b->second, p});
+                c->kept_bytes += b->second;
+                continue;
+            }
+            if (b != c->block_size.end()) c->block_size.erase(b);
+            (void)hipFree(p);
+        }
     }
     allocs.clear();
     c->used -= std::min<uint64_t>(c->used, bytes);
@@ -234,17 +278,18 @@ size_t psi_floats(const Model& m, int f)
     return ax == 2 ? (size_t)(P.ps2 * 2 * m.g.npml) : (size_t)(P.ps2 * n3[2]);
 }
 
-int alloc_state(gpi_ctx* c, const Model& m, State* st)
+int alloc_state(gpi_ctx* c, const Model& m, State* st, bool reuse)
 {
     for (int f = GPI_P; f <= GPI_TAUYZ; ++f) {
         if (!field_codes(m.g.ndim, m.g.physics, f)) continue;
-        int rc = dev_alloc(c, &st->allocs, &st->bytes, (void**)&st->field[f], sizeof(float) * (size_t)m.slab);
+        int rc = dev_alloc(c, &st->allocs, &st->bytes, (void**)&st->field[f], sizeof(float) * (size_t)m.slab,
+                           reuse);
         if (rc) return rc;
     }
     for (int f = GPI_DPDX; f < GPI_NFIELDS; ++f) {
         const size_t n = psi_floats(m, f);
         if (!n) continue;
-        int rc = dev_alloc(c, &st->allocs, &st->bytes, (void**)&st->psi[f], sizeof(float) * n);
+        int rc = dev_alloc(c, &st->allocs, &st->bytes, (void**)&st->psi[f], sizeof(float) * n, reuse);
         if (rc) return rc;
     }
     return GPI_OK;
@@ -259,9 +304,13 @@ int zero_state(gpi_ctx* c, const Model& m, const State& st, hipStream_t s)
     return GPI_OK;
 }
 
+// Uploads up to here go through the context's pinned ring without waiting for the copy.
+static constexpr size_t SMALL_UPLOAD = (size_t)256 << 10;
+
 int copy_h2d(gpi_ctx* c, void* dst, const void* src, size_t bytes)
 {
     PinnedStage* st = c->stage;
+    if (!st && c->keep_cap && bytes <= SMALL_UPLOAD) st = &c->small;
     if (!st) {
         HIPTRY(c, hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
         return GPI_OK;
@@ -273,7 +322,7 @@ int copy_h2d(gpi_ctx* c, void* dst, const void* src, size_t bytes)
         if (st->buf) (void)hipHostFree(st->buf);
         st->buf = nullptr;
         st->cap = st->off = 0;
-        const size_t cap = std::max<size_t>(need, (size_t)64 << 20);
+        const size_t cap = std::max<size_t>(need, st == &c->small ? 16 * SMALL_UPLOAD : (size_t)64 << 20);
         HIPTRY(c, hipHostMalloc((void**)&st->buf, cap, hipHostMallocDefault));
         st->cap = cap;
     } else if (st->off + need > st->cap) {   // wrap once every queued copy has finished
