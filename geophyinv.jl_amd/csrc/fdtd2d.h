@@ -18,6 +18,7 @@ struct VelParams2D {
     int gx, gy;        // stencil workgroups along z and x
     uint32_t pml_mask, rigid_mask;
     float dxI, dzI, dt;
+    int64_t out;       // the updated velocities go `out` floats behind those read
 };
 
 struct StrParams2D {
@@ -35,6 +36,7 @@ struct StrParams2D {
     int gx, gy;
     uint32_t pml_mask, free_mask;
     float dxI, dzI;
+    int64_t out;       // the updated stresses go `out` floats behind those read
 };
 
 // Injection buckets (64-row segment of one derivative-grid column): bucket of point (i, j)

@@ -102,7 +102,7 @@ __device__ __forceinline__ void load_x(float (&v)[O], const float* a, int off, i
 // Each point function first issues every load its updates need (no store precedes them,
 // so they go out together), then evaluates and stores in the reference's order.
 
-template <int O>
+template <int O, bool RING>
 __device__ __forceinline__ void vel_ac_point(const VelParams2D& P, const PassExtras& X, int64_t it, int ninj, int i,
                                              int j)
 {
@@ -134,24 +134,24 @@ __device__ __forceinline__ void vel_ac_point(const VelParams2D& P, const PassExt
         float nv = vxo + cxo * d;
         // rigid x faces: the only nonzero ghost mirrors the first/last interior column
         // (dirichlet.jl ighostmin/ighostmax with ifd = 1), taken before the source term
-        if ((P.rigid_mask & GPI_FACE(2, 0)) && j == 0) P.vx[(i + H)] = -nv;
-        if ((P.rigid_mask & GPI_FACE(2, 1)) && j == P.nx - H - 1) P.vx[(i + H) + ld * (P.nx + H - 1)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(2, 0)) && j == 0) into<RING>(P.vx, P.out)[(i + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(2, 1)) && j == P.nx - H - 1) into<RING>(P.vx, P.out)[(i + H) + ld * (P.nx + H - 1)] = -nv;
         if (ninj) nv = inject_velocity(X, it, INJ_VX, bk, o, nv, P.rho, P.dt);
-        P.vx[o] = nv;
+        into<RING>(P.vx, P.out)[o] = nv;
     }
     // vz[inn] += dtinvavzirho * dpdz, dpdz = D_zi(p) * dzI
     if (uz) {
         float d = stencil<O>(pz) * P.dzI;
         d = cpml_z(d, P.qz0, i, j, P.npml, P.pml_mask);
         float nv = vzo + czo * d;
-        if ((P.rigid_mask & GPI_FACE(0, 0)) && i == 0) P.vz[ld * (j + H)] = -nv;
-        if ((P.rigid_mask & GPI_FACE(0, 1)) && i == P.nz - H - 1) P.vz[(P.nz + H - 1) + ld * (j + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(0, 0)) && i == 0) into<RING>(P.vz, P.out)[ld * (j + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(0, 1)) && i == P.nz - H - 1) into<RING>(P.vz, P.out)[(P.nz + H - 1) + ld * (j + H)] = -nv;
         if (ninj) nv = inject_velocity(X, it, INJ_VZ, bk, o, nv, P.rho, P.dt);
-        P.vz[o] = nv;
+        into<RING>(P.vz, P.out)[o] = nv;
     }
 }
 
-template <int O>
+template <int O, bool RING>
 __device__ __forceinline__ void str_ac_point(const StrParams2D& P, const PassExtras& X, int64_t it, int ninj, int i,
                                              int j)
 {
@@ -175,7 +175,7 @@ __device__ __forceinline__ void str_ac_point(const StrParams2D& P, const PassExt
         int t;
         if (X.inj[q].kind == INJ_P && injection_sum(X.inj[q], bk, o, it, acc, t)) p = p + (acc * c);
     }
-    P.s0[o] = p;
+    into<RING>(P.s0, P.out)[o] = p;
 }
 
 // Elastic updates from their operands (the point functions below load them).
@@ -242,7 +242,7 @@ __device__ __forceinline__ float str_el_shear(const StrParams2D& P, int i, int j
     return s2o - c2o * (a + c);
 }
 
-template <int O>
+template <int O, bool RING>
 __device__ __forceinline__ void vel_el_point(const VelParams2D& P, const PassExtras& X, int64_t it, int ninj, int i,
                                              int j)
 {
@@ -271,21 +271,21 @@ __device__ __forceinline__ void vel_el_point(const VelParams2D& P, const PassExt
     const float czo = dt_over_av2(P.dt, rz0, rz1);   // dtinvavzirho
     if (ux) {
         float nv = vel_el_vx<O>(P, i, j, a1, a2, vxo, cxo);
-        if ((P.rigid_mask & GPI_FACE(2, 0)) && j == 0) P.vx[(i + H)] = -nv;
-        if ((P.rigid_mask & GPI_FACE(2, 1)) && j == P.nx - H - 1) P.vx[(i + H) + ld * (P.nx + H - 1)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(2, 0)) && j == 0) into<RING>(P.vx, P.out)[(i + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(2, 1)) && j == P.nx - H - 1) into<RING>(P.vx, P.out)[(i + H) + ld * (P.nx + H - 1)] = -nv;
         if (ninj) nv = inject_velocity(X, it, INJ_VX, bk, o, nv, P.rho, P.dt);
-        P.vx[o] = nv;
+        into<RING>(P.vx, P.out)[o] = nv;
     }
     if (uz) {
         float nv = vel_el_vz<O>(P, i, j, b1, b2, vzo, czo);
-        if ((P.rigid_mask & GPI_FACE(0, 0)) && i == 0) P.vz[ld * (j + H)] = -nv;
-        if ((P.rigid_mask & GPI_FACE(0, 1)) && i == P.nz - H - 1) P.vz[(P.nz + H - 1) + ld * (j + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(0, 0)) && i == 0) into<RING>(P.vz, P.out)[ld * (j + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(0, 1)) && i == P.nz - H - 1) into<RING>(P.vz, P.out)[(P.nz + H - 1) + ld * (j + H)] = -nv;
         if (ninj) nv = inject_velocity(X, it, INJ_VZ, bk, o, nv, P.rho, P.dt);
-        P.vz[o] = nv;
+        into<RING>(P.vz, P.out)[o] = nv;
     }
 }
 
-template <int O>
+template <int O, bool RING>
 __device__ __forceinline__ void str_el_point(const StrParams2D& P, const PassExtras& X, int64_t it, int ninj, int i,
                                              int j)
 {
@@ -321,14 +321,14 @@ __device__ __forceinline__ void str_el_point(const StrParams2D& P, const PassExt
         float txx, tzz;
         str_el_normal<O>(P, i, j, ax, az, s0o, s1o, m, l, txx, tzz);
         // free surface at zmin, before the sources: tauzz[1,:] = -tauzz[2,:]
-        if (fs && i == 1) P.s1[ld * j] = -tzz;
+        if (fs && i == 1) into<RING>(P.s1, P.out)[ld * j] = -tzz;
         if (ninj) inject_normal2(X, it, ninj, (i >> 6) + P.gx * j, o, m, txx, tzz);
-        P.s0[o] = txx;
-        if (!(fs && i == 0)) P.s1[o] = tzz;
+        into<RING>(P.s0, P.out)[o] = txx;
+        if (!(fs && i == 0)) into<RING>(P.s1, P.out)[o] = tzz;
     }
     if (us) {
         const float t = str_el_shear<O>(P, i, j, bz, bx, s2o, c2o);
-        P.s2[o] = (fs && i == 0) ? 0.0f : t;         // tauxz[1,:] = 0
+        into<RING>(P.s2, P.out)[o] = (fs && i == 0) ? 0.0f : t;         // tauxz[1,:] = 0
     }
 }
 
@@ -338,27 +338,27 @@ __device__ __forceinline__ void str_el_point(const StrParams2D& P, const PassExt
 // TY*RX*(b / gx)..
 // ---------------------------------------------------------------------------------------
 
-template <int O, int PHYS, int TY, int RX>
+template <int O, int PHYS, int TY, int RX, bool RING>
 __device__ __forceinline__ void vel_tile(const VelParams2D& P, const PassExtras& X, int64_t it, int ninj, int b)
 {
     const int i = (b % P.gx) * 64 + (int)threadIdx.x;
     const int j0 = (b / P.gx) * (TY * RX) + (int)threadIdx.y * RX;
 #pragma unroll
     for (int r = 0; r < RX; ++r) {
-        if (PHYS == 0) vel_ac_point<O>(P, X, it, ninj, i, j0 + r);
-        else vel_el_point<O>(P, X, it, ninj, i, j0 + r);
+        if (PHYS == 0) vel_ac_point<O, RING>(P, X, it, ninj, i, j0 + r);
+        else vel_el_point<O, RING>(P, X, it, ninj, i, j0 + r);
     }
 }
 
-template <int O, int PHYS, int TY, int RX>
+template <int O, int PHYS, int TY, int RX, bool RING>
 __device__ __forceinline__ void str_tile(const StrParams2D& P, const PassExtras& X, int64_t it, int ninj, int b)
 {
     const int i = (b % P.gx) * 64 + (int)threadIdx.x;
     const int j0 = (b / P.gx) * (TY * RX) + (int)threadIdx.y * RX;
 #pragma unroll
     for (int r = 0; r < RX; ++r) {
-        if (PHYS == 0) str_ac_point<O>(P, X, it, ninj, i, j0 + r);
-        else str_el_point<O>(P, X, it, ninj, i, j0 + r);
+        if (PHYS == 0) str_ac_point<O, RING>(P, X, it, ninj, i, j0 + r);
+        else str_el_point<O, RING>(P, X, it, ninj, i, j0 + r);
     }
 }
 
@@ -379,7 +379,7 @@ int plain_shape()
     return t;
 }
 
-template <int O, int PHYS, int TY, int RX>
+template <int O, int PHYS, int TY, int RX, bool RING>
 __global__ __launch_bounds__(64 * TY) void vel2d_kernel(VelParams2D P, PassExtras X)
 {
     const int b = xcd_remap(blockIdx.x, gridDim.x);
@@ -388,10 +388,10 @@ __global__ __launch_bounds__(64 * TY) void vel2d_kernel(VelParams2D P, PassExtra
         gather_block<4>(X, X.it, b - nbm);
         return;
     }
-    vel_tile<O, PHYS, TY, RX>(P, X, X.it, X.ninj, b);
+    vel_tile<O, PHYS, TY, RX, RING>(P, X, X.it, X.ninj, b);
 }
 
-template <int O, int PHYS, int TY, int RX>
+template <int O, int PHYS, int TY, int RX, bool RING>
 __global__ __launch_bounds__(64 * TY) void str2d_kernel(StrParams2D P, PassExtras X)
 {
     const int b = xcd_remap(blockIdx.x, gridDim.x);
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(64 * TY) void str2d_kernel(StrParams2D P, PassExtra
         gather_block<4>(X, X.it, b - nbm);
         return;
     }
-    str_tile<O, PHYS, TY, RX>(P, X, X.it, X.ninj, b);
+    str_tile<O, PHYS, TY, RX, RING>(P, X, X.it, X.ninj, b);
 }
 
 template <int O, int PHYS, int TY, int RX>
@@ -410,13 +410,15 @@ void launch_plain(bool velocity, hipStream_t s, VelParams2D V, StrParams2D S, co
     if (velocity) {
         V.gx = (V.nz - H + 63) / 64;
         V.gy = (V.nx - H + TY * RX - 1) / (TY * RX);
-        hipLaunchKernelGGL((vel2d_kernel<O, PHYS, TY, RX>), dim3(V.gx * V.gy + X.gather_blocks), dim3(64, TY), 0, s,
-                           V, X);
+        const dim3 grd(V.gx * V.gy + X.gather_blocks), blk(64, TY);
+        if (V.out) hipLaunchKernelGGL((vel2d_kernel<O, PHYS, TY, RX, true>), grd, blk, 0, s, V, X);
+        else hipLaunchKernelGGL((vel2d_kernel<O, PHYS, TY, RX, false>), grd, blk, 0, s, V, X);
     } else {
         S.gx = (S.nz + 63) / 64;
         S.gy = (S.nx + TY * RX - 1) / (TY * RX);
-        hipLaunchKernelGGL((str2d_kernel<O, PHYS, TY, RX>), dim3(S.gx * S.gy + X.gather_blocks), dim3(64, TY), 0, s,
-                           S, X);
+        const dim3 grd(S.gx * S.gy + X.gather_blocks), blk(64, TY);
+        if (S.out) hipLaunchKernelGGL((str2d_kernel<O, PHYS, TY, RX, true>), grd, blk, 0, s, S, X);
+        else hipLaunchKernelGGL((str2d_kernel<O, PHYS, TY, RX, false>), grd, blk, 0, s, S, X);
     }
 }
 
@@ -484,7 +486,7 @@ __device__ __forceinline__ void vel_batch_block(const BatchShot2D* __restrict__ 
         if (it < S.nt) gather_block<4>(S.xv, it, lb - nbm);
         return;
     }
-    vel_tile<O, PHYS, TY, RX>(S.vp, S.xv, it, it < S.nt ? S.xv.ninj : 0, lb);
+    vel_tile<O, PHYS, TY, RX, false>(S.vp, S.xv, it, it < S.nt ? S.xv.ninj : 0, lb);
 }
 
 template <int O, int PHYS, int TY, int RX>
@@ -502,7 +504,7 @@ __device__ __forceinline__ void str_batch_block(const BatchShot2D* __restrict__ 
         gather_block<4>(S.xs, it, lb - nbm);
         return;
     }
-    str_tile<O, PHYS, TY, RX>(S.sp, S.xs, it, S.xs.ninj, lb);
+    str_tile<O, PHYS, TY, RX, false>(S.sp, S.xs, it, S.xs.ninj, lb);
 }
 
 template <int O, int PHYS, int TY, int RX>
@@ -608,6 +610,7 @@ bool vel_params_2d(const Model& m, const State& st, VelParams2D* out)
     P.s2 = ac ? nullptr : st.field[GPI_TAUXZ];
     P.vx = st.field[GPI_VX];
     P.vz = st.field[GPI_VZ];
+    P.out = st.vout;
     P.rho = m.coef[GPI_C_RHO];
     P.qx0 = pml_of(m, st, ac ? GPI_DPDX : GPI_DTAUXXDX);
     P.qx1 = ac ? Pml{} : pml_of(m, st, GPI_DTAUXZDX);
@@ -638,6 +641,7 @@ bool str_params_2d(const Model& m, const State& st, StrParams2D* out)
     P.s0 = st.field[ac ? GPI_P : GPI_TAUXX];
     P.s1 = ac ? nullptr : st.field[GPI_TAUZZ];
     P.s2 = ac ? nullptr : st.field[GPI_TAUXZ];
+    P.out = st.sout;
     P.c0 = m.coef[ac ? GPI_C_DTK : GPI_C_INVLAMBDA];
     P.c1 = ac ? nullptr : m.coef[GPI_C_INVMU];
     P.dt = m.g.dt;

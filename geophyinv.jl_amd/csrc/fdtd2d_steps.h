@@ -52,6 +52,11 @@ struct StepParams2D {
     float dxI, dzI, dt;
     int lead;                // halo cells on each side of a tile
     int steps;               // time steps of this launch (lead >= steps * h)
+    // arrays that keep every step (their `in` and `out` are slots hstart and hstart + steps): the
+    // ring's first slot, else null
+    float* hist[5];
+    int64_t hslab;
+    int hslots, hstart;
     int ntile;
     const TileBox* box;
     int64_t it0;
@@ -81,7 +86,8 @@ struct StepPlan {
 int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& src,
                   const gpi_shot* shot, const std::vector<DevPoints>& rec, StepPlan* plan,
                   bool* ok);
-// `steps` <= plan.steps time steps from it0
-void run_steps_2d(const Model& m, StepPlan& plan, int64_t it0, int steps, hipStream_t s);
+// `steps` <= plan.steps time steps from it0; the arrays of `ring` (if given) take the slots
+// after its current one instead of the two states
+void run_steps_2d(const Model& m, StepPlan& plan, int64_t it0, int steps, hipStream_t s, Ring* ring = nullptr);
 
 }  // namespace gpi

@@ -28,6 +28,7 @@ struct VelParams3D {
     int xfast;         // elastic: consecutive workgroups walk along x (then z, y tiles)
     uint32_t pml_mask, rigid_mask;
     float dxI, dyI, dzI, dt;
+    int64_t out;       // the updated velocities go `out` floats behind those read
 };
 
 struct StrParams3D {
@@ -51,6 +52,7 @@ struct StrParams3D {
     int xfast;         // elastic: consecutive workgroups walk along x (then z, y tiles)
     uint32_t pml_mask, free_mask;
     float dxI, dyI, dzI;
+    int64_t out;       // the updated stresses go `out` floats behind those read
 };
 
 // Rows of the 3-D velocity passes are shifted by h: workgroup row bx covers

@@ -175,7 +175,7 @@ __device__ __forceinline__ int decode(int b, int gx, int gy, int nk, bool xfast,
 // instead of once per plane that uses it.  The injection bucket of a point is the
 // per-plane tile id bx + gx*(by + gy*k), as planned on the host.
 
-template <int O, bool NT>
+template <int O, bool NT, bool RING>
 __global__ __launch_bounds__(512) void vel3d_acoustic(VelParams3D P, PassExtras X)
 {
     constexpr int H = O - 1;
@@ -245,33 +245,33 @@ __global__ __launch_bounds__(512) void vel3d_acoustic(VelParams3D P, PassExtras 
             float d = stencil<O>(w) * P.dxI;
             d = cpml3_x<false>(d, P.qx[0], iu, ju, k, P.npml, P.pml_mask);
             float nv = cur.vxo + cur.cxo * d;
-            if ((P.rigid_mask & GPI_FACE(2, 0)) && k == 0) P.vx[(iu + H) + s1 * (ju + H)] = -nv;
+            if ((P.rigid_mask & GPI_FACE(2, 0)) && k == 0) into<RING>(P.vx, P.out)[(iu + H) + s1 * (ju + H)] = -nv;
             if ((P.rigid_mask & GPI_FACE(2, 1)) && k == P.nx - H - 1)
-                P.vx[(iu + H) + s1 * (ju + H) + s2 * (P.nx + H - 1)] = -nv;
+                into<RING>(P.vx, P.out)[(iu + H) + s1 * (ju + H) + s2 * (P.nx + H - 1)] = -nv;
             if (X.ninj) nv = inject_velocity(X, INJ_VX, bt, o, nv, P.rho, P.dt);
-            store_out<NT>(&P.vx[o], nv);
+            store_out<NT>(&into<RING>(P.vx, P.out)[o], nv);
         }
         // vy on (nz-2h, ny-h, nx-2h): dpdy = D_yi(p)
         if (ycol && k < P.nx - 2 * H) {
             float d = stencil<O>(cur.py) * P.dyI;
             d = cpml3_y<false>(d, P.qy[0], iu, ju, k, P.npml, P.pml_mask);
             float nv = cur.vyo + cur.cyo * d;
-            if ((P.rigid_mask & GPI_FACE(1, 0)) && ju == 0) P.vy[(iu + H) + s2 * (k + H)] = -nv;
+            if ((P.rigid_mask & GPI_FACE(1, 0)) && ju == 0) into<RING>(P.vy, P.out)[(iu + H) + s2 * (k + H)] = -nv;
             if ((P.rigid_mask & GPI_FACE(1, 1)) && ju == P.ny - H - 1)
-                P.vy[(iu + H) + s1 * (P.ny + H - 1) + s2 * (k + H)] = -nv;
+                into<RING>(P.vy, P.out)[(iu + H) + s1 * (P.ny + H - 1) + s2 * (k + H)] = -nv;
             if (X.ninj) nv = inject_velocity(X, INJ_VY, bt, o, nv, P.rho, P.dt);
-            store_out<NT>(&P.vy[o], nv);
+            store_out<NT>(&into<RING>(P.vy, P.out)[o], nv);
         }
         // vz on (nz-h, ny-2h, nx-2h): dpdz = D_zi(p)
         if (zcol && k < P.nx - 2 * H) {
             float d = stencil<O>(cur.pz) * P.dzI;
             d = cpml3_z<false>(d, P.qz[0], iu, ju, k, P.npml, P.pml_mask);
             float nv = cur.vzo + cur.czo * d;
-            if ((P.rigid_mask & GPI_FACE(0, 0)) && iu == 0) P.vz[s1 * (ju + H) + s2 * (k + H)] = -nv;
+            if ((P.rigid_mask & GPI_FACE(0, 0)) && iu == 0) into<RING>(P.vz, P.out)[s1 * (ju + H) + s2 * (k + H)] = -nv;
             if ((P.rigid_mask & GPI_FACE(0, 1)) && iu == P.nz - H - 1)
-                P.vz[(P.nz + H - 1) + s1 * (ju + H) + s2 * (k + H)] = -nv;
+                into<RING>(P.vz, P.out)[(P.nz + H - 1) + s1 * (ju + H) + s2 * (k + H)] = -nv;
             if (X.ninj) nv = inject_velocity(X, INJ_VZ, bt, o, nv, P.rho, P.dt);
-            store_out<NT>(&P.vz[o], nv);
+            store_out<NT>(&into<RING>(P.vz, P.out)[o], nv);
         }
     };
     // two planes per trip with alternating operand sets: no register whose load may be
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(512) void vel3d_acoustic(VelParams3D P, PassExtras 
     }
 }
 
-template <int O, bool NT>
+template <int O, bool NT, bool RING>
 __global__ __launch_bounds__(512) void str3d_acoustic(StrParams3D P, PassExtras X)
 {
     const int b = tile_order((int)blockIdx.x, (int)gridDim.x, P.remap);
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(512) void str3d_acoustic(StrParams3D P, PassExtras 
             int tt;
             if (X.inj[q].kind == INJ_P && injection_sum(X.inj[q], bt, o, X.it, acc, tt)) pn = pn + (acc * c);
         }
-        store_out<NT>(&P.s[0][o], pn);
+        store_out<NT>(&into<RING>(P.s[0], P.out)[o], pn);
         cur = nxt;
     }
 }
@@ -370,7 +370,7 @@ struct VelElSamples {
     float e1, e2, e3;                    // D_xa(tauxz), D_ya(tauyz), D_zi(tauzz)
 };
 
-template <int O>
+template <int O, bool RING>
 __device__ __forceinline__ void vel3d_elastic_update(const VelParams3D& P, const PassExtras& X, int i, int j, int k,
                                                      int bt, int o, bool ux, bool uy, bool uz, const VelElSamples& v)
 {
@@ -385,11 +385,11 @@ __device__ __forceinline__ void vel3d_elastic_update(const VelParams3D& P, const
         const float d2 = cpml3_y(v.a2, P.qy[0], i, j, k, P.npml, P.pml_mask);
         const float d3 = cpml3_z(v.a3, P.qz[0], i, j, k, P.npml, P.pml_mask);
         float nv = v.vxo - cxo * ((d1 + d2) + d3);
-        if ((P.rigid_mask & GPI_FACE(2, 0)) && k == 0) P.vx[(i + H) + s1 * (j + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(2, 0)) && k == 0) into<RING>(P.vx, P.out)[(i + H) + s1 * (j + H)] = -nv;
         if ((P.rigid_mask & GPI_FACE(2, 1)) && k == P.nx - H - 1)
-            P.vx[(i + H) + s1 * (j + H) + s2 * (P.nx + H - 1)] = -nv;
+            into<RING>(P.vx, P.out)[(i + H) + s1 * (j + H) + s2 * (P.nx + H - 1)] = -nv;
         if (X.ninj) nv = inject_velocity(X, INJ_VX, bt, o, nv, P.rho, P.dt);
-        P.vx[o] = nv;
+        into<RING>(P.vx, P.out)[o] = nv;
     }
     // vy -= dtinvavyirho*((dtauxydx + dtauyydy) + dtauyzdz) on (nz-2h, ny-h, nx-2h)
     if (uy) {
@@ -397,11 +397,11 @@ __device__ __forceinline__ void vel3d_elastic_update(const VelParams3D& P, const
         const float d2 = cpml3_y(v.b2, P.qy[1], i, j, k, P.npml, P.pml_mask);
         const float d3 = cpml3_z(v.b3, P.qz[1], i, j, k, P.npml, P.pml_mask);
         float nv = v.vyo - cyo * ((d1 + d2) + d3);
-        if ((P.rigid_mask & GPI_FACE(1, 0)) && j == 0) P.vy[(i + H) + s2 * (k + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(1, 0)) && j == 0) into<RING>(P.vy, P.out)[(i + H) + s2 * (k + H)] = -nv;
         if ((P.rigid_mask & GPI_FACE(1, 1)) && j == P.ny - H - 1)
-            P.vy[(i + H) + s1 * (P.ny + H - 1) + s2 * (k + H)] = -nv;
+            into<RING>(P.vy, P.out)[(i + H) + s1 * (P.ny + H - 1) + s2 * (k + H)] = -nv;
         if (X.ninj) nv = inject_velocity(X, INJ_VY, bt, o, nv, P.rho, P.dt);
-        P.vy[o] = nv;
+        into<RING>(P.vy, P.out)[o] = nv;
     }
     // vz -= dtinvavzirho*((dtauxzdx + dtauyzdy) + dtauzzdz) on (nz-h, ny-2h, nx-2h)
     if (uz) {
@@ -409,16 +409,16 @@ __device__ __forceinline__ void vel3d_elastic_update(const VelParams3D& P, const
         const float d2 = cpml3_y(v.e2, P.qy[2], i, j, k, P.npml, P.pml_mask);
         const float d3 = cpml3_z(v.e3, P.qz[2], i, j, k, P.npml, P.pml_mask);
         float nv = v.vzo - czo * ((d1 + d2) + d3);
-        if ((P.rigid_mask & GPI_FACE(0, 0)) && i == 0) P.vz[s1 * (j + H) + s2 * (k + H)] = -nv;
+        if ((P.rigid_mask & GPI_FACE(0, 0)) && i == 0) into<RING>(P.vz, P.out)[s1 * (j + H) + s2 * (k + H)] = -nv;
         if ((P.rigid_mask & GPI_FACE(0, 1)) && i == P.nz - H - 1)
-            P.vz[(P.nz + H - 1) + s1 * (j + H) + s2 * (k + H)] = -nv;
+            into<RING>(P.vz, P.out)[(P.nz + H - 1) + s1 * (j + H) + s2 * (k + H)] = -nv;
         if (X.ninj) nv = inject_velocity(X, INJ_VZ, bt, o, nv, P.rho, P.dt);
-        P.vz[o] = nv;
+        into<RING>(P.vz, P.out)[o] = nv;
     }
 }
 
 // One (z, y) point of plane k of the elastic velocity pass; bt is the injection bucket.
-template <int O>
+template <int O, bool RING>
 __device__ __forceinline__ void vel3d_elastic_point(const VelParams3D& P, const PassExtras& X, int i, int j, int k,
                                                     int bt)
 {
@@ -477,7 +477,7 @@ __device__ __forceinline__ void vel3d_elastic_point(const VelParams3D& P, const 
         v.e2 = stencil<O>(e2) * P.dyI;
         v.e3 = stencil<O>(e3) * P.dzI;
     }
-    vel3d_elastic_update<O>(P, X, i, j, k, bt, o, ux, uy, uz, v);
+    vel3d_elastic_update<O, RING>(P, X, i, j, k, bt, o, ux, uy, uz, v);
 }
 
 // Elastic workgroups are 64 (z) x TY (y) x KZ (x) threads: the layer threadIdx.z of
@@ -486,7 +486,7 @@ __device__ __forceinline__ void vel3d_elastic_point(const VelParams3D& P, const 
 // served by its CU's caches rather than fetched again by another workgroup later (as a
 // loop over planes would do, but without the registers the compiler keeps live across
 // such a loop).  With KZ = 1 the xfast order is available as before.
-template <int O>
+template <int O, bool RING>
 __global__ __launch_bounds__(512) void vel3d_elastic(VelParams3D P, PassExtras X)
 {
     constexpr int H = O - 1;
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(512) void vel3d_elastic(VelParams3D P, PassExtras X
     Idx3 t;
     const int bt = decode(b, P.gx, P.gy, nch, P.xfast != 0, t);
     if (t.k >= nxw) return;
-    vel3d_elastic_point<O>(P, X, t.i - H, t.j, t.k, bt);   // rows shifted by h
+    vel3d_elastic_point<O, RING>(P, X, t.i - H, t.j, t.k, bt);   // rows shifted by h
 }
 
 // The elastic stress update of point (i, j, k) from its derivative samples (stencil times
@@ -518,7 +518,7 @@ struct StrElSamples {
 };
 
 // ZP: the caller has applied the derivatives' z-CPML (the staged pass, from its own loads).
-template <int O, bool ZP = false>
+template <int O, bool RING, bool ZP = false>
 __device__ __forceinline__ void str3d_elastic_update(const StrParams3D& P, const PassExtras& X, int i, int j, int k,
                                                      int bt, int o, bool un, bool uxz, bool uxy, bool uyz,
                                                      const StrElSamples& v)
@@ -538,7 +538,7 @@ __device__ __forceinline__ void str3d_elastic_update(const StrParams3D& P, const
         float txx = (v.s0 - (m * dvx)) - (l * (dvy + dvz));
         float tyy = (v.s1 - (m * dvy)) - (l * (dvx + dvz));
         float tzz = (v.s2 - (m * dvz)) - (l * (dvy + dvx));
-        if (fs && i == 1) P.s[2][s1 * j + s2 * k] = -tzz;   // tauzz[1,:,:] = -tauzz[2,:,:]
+        if (fs && i == 1) into<RING>(P.s[2], P.out)[s1 * j + s2 * k] = -tzz;   // tauzz[1,:,:] = -tauzz[2,:,:]
         for (int q = 0; q < X.ninj; ++q) {
             float acc;
             int tt;
@@ -548,34 +548,34 @@ __device__ __forceinline__ void str3d_elastic_update(const StrParams3D& P, const
                 tzz = tzz + (acc * m);
             }
         }
-        P.s[0][o] = txx;
-        P.s[1][o] = tyy;
-        if (!(fs && i == 0)) P.s[2][o] = tzz;
+        into<RING>(P.s[0], P.out)[o] = txx;
+        into<RING>(P.s[1], P.out)[o] = tyy;
+        if (!(fs && i == 0)) into<RING>(P.s[2], P.out)[o] = tzz;
     }
     // tauxz -= dtavxzimu*(dvxdz + dvzdx) on (nz-h, ny-2h, nx-h)
     if (uxz) {
         const float a = ZP ? v.xza : cpml3_z(v.xza, P.qz[1], i, j, k, P.npml, P.pml_mask);
         const float c = cpml3_x(v.xzc, P.qx[2], i, j, k, P.npml, P.pml_mask);
         const float r = v.s4 - c3o * (a + c);
-        P.s[4][o] = (fs && i == 0) ? 0.0f : r;
+        into<RING>(P.s[4], P.out)[o] = (fs && i == 0) ? 0.0f : r;
     }
     // tauxy -= dtavxyimu*(dvxdy + dvydx) on (nz-2h, ny-h, nx-h)
     if (uxy) {
         const float a = cpml3_y(v.xya, P.qy[1], i, j, k, P.npml, P.pml_mask);
         const float c = cpml3_x(v.xyc, P.qx[1], i, j, k, P.npml, P.pml_mask);
-        P.s[3][o] = v.s3 - c2o * (a + c);
+        into<RING>(P.s[3], P.out)[o] = v.s3 - c2o * (a + c);
     }
     // tauyz -= dtavyzimu*(dvydz + dvzdy) on (nz-h, ny-h, nx-2h)
     if (uyz) {
         const float a = ZP ? v.yza : cpml3_z(v.yza, P.qz[2], i, j, k, P.npml, P.pml_mask);
         const float c = cpml3_y(v.yzc, P.qy[2], i, j, k, P.npml, P.pml_mask);
         const float r = v.s5 - c4o * (a + c);
-        P.s[5][o] = (fs && i == 0) ? 0.0f : r;
+        into<RING>(P.s[5], P.out)[o] = (fs && i == 0) ? 0.0f : r;
     }
 }
 
 // One (z, y) point of plane k of the elastic stress pass; bt is the injection bucket.
-template <int O>
+template <int O, bool RING>
 __device__ __forceinline__ void str3d_elastic_point(const StrParams3D& P, const PassExtras& X, int i, int j, int k,
                                                     int bt)
 {
@@ -649,10 +649,10 @@ __device__ __forceinline__ void str3d_elastic_point(const StrParams3D& P, const 
         v.yza = stencil<O>(yz1) * P.dzI;
         v.yzc = stencil<O>(yz2) * P.dyI;
     }
-    str3d_elastic_update<O>(P, X, i, j, k, bt, o, un, uxz, uxy, uyz, v);
+    str3d_elastic_update<O, RING>(P, X, i, j, k, bt, o, un, uxz, uxy, uyz, v);
 }
 
-template <int O>
+template <int O, bool RING>
 __global__ __launch_bounds__(512) void str3d_elastic(StrParams3D P, PassExtras X)
 {
     const int b = P.remap ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(512) void str3d_elastic(StrParams3D P, PassExtras X
     Idx3 t;
     const int bt = decode(b, P.gx, P.gy, nch, P.xfast != 0, t);
     if (t.k >= P.nx) return;
-    str3d_elastic_point<O>(P, X, t.i, t.j, t.k, bt);
+    str3d_elastic_point<O, RING>(P, X, t.i, t.j, t.k, bt);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -816,7 +816,7 @@ __device__ __forceinline__ float lds_y(const float* L, int r, int c)
     return stencil<O>(v);
 }
 
-template <int O, int TY>
+template <int O, int TY, bool RING>
 __global__ __launch_bounds__(64 * TY) void vel3d_elastic_staged(VelParams3D P, PassExtras X)
 {
     constexpr int H = O - 1;
@@ -919,7 +919,7 @@ __global__ __launch_bounds__(64 * TY) void vel3d_elastic_staged(VelParams3D P, P
             v.e3 = lds_z<O, W>(Lzz, ty + H, tx) * P.dzI;   // D_zi(tauzz) at (i, j+h, k+h)
             const int bt = bx + P.gx * (by + P.gy * k);
             const int io = opaque(i), jo = __builtin_amdgcn_readfirstlane(opaque(j));
-            vel3d_elastic_update<O>(P, X, io, jo, k, bt, (io + H) + s1 * (jo + H) + s2 * p, ux, uy, uz, v);
+            vel3d_elastic_update<O, RING>(P, X, io, jo, k, bt, (io + H) + s1 * (jo + H) + s2 * p, ux, uy, uz, v);
         }
         if (p < plast) {   // plane p+1 (loaded) into the other slot; loads for the next planes
 #pragma unroll
@@ -930,8 +930,9 @@ __global__ __launch_bounds__(64 * TY) void vel3d_elastic_staged(VelParams3D P, P
     }
 }
 
-template <int O, int TY, bool ZP>
-__global__ __launch_bounds__(64 * TY) void str3d_elastic_staged(StrParams3D P, PassExtras X)
+// order 2: six waves per SIMD (80 registers; 81 in the ring form without the bound)
+template <int O, int TY, bool ZP, bool RING>
+__global__ __launch_bounds__(64 * TY, (O == 2 ? 6 : 1)) void str3d_elastic_staged(StrParams3D P, PassExtras X)
 {
     constexpr int H = O - 1;
     using S = PlaneStage<TY, H, 0, 64>;
@@ -1054,7 +1055,7 @@ __global__ __launch_bounds__(64 * TY) void str3d_elastic_staged(StrParams3D P, P
                 v.xza = zstrip_apply(v.xza, zm[1], Lz, 1, P.qz[1], io, jo, k, P.npml, P.pml_mask, uxz);
                 v.yza = zstrip_apply(v.yza, zm[2], Lz, 2, P.qz[2], io, jo, k, P.npml, P.pml_mask, uyz);
             }
-            str3d_elastic_update<O, ZP>(P, X, io, jo, k, bt, io + s1 * jo + s2 * k, un, uxz, uxy, uyz, v);
+            str3d_elastic_update<O, RING, ZP>(P, X, io, jo, k, bt, io + s1 * jo + s2 * k, un, uxz, uxy, uyz, v);
         }
         if (p < plast) {   // plane p+1 (loaded) into the other slot; loads for the next planes
 #pragma unroll
@@ -1199,7 +1200,7 @@ bool elastic_xfast()
     return e == 1;
 }
 
-template <int O>
+template <int O, bool RING>
 void launch_vel3(const Model& m, hipStream_t s, VelParams3D P, const PassExtras& X)
 {
     constexpr int H = O - 1;
@@ -1210,9 +1211,9 @@ void launch_vel3(const Model& m, hipStream_t s, VelParams3D P, const PassExtras&
         P.kc = elastic_march(P.nx - H);
         P.remap = elastic_window() ? std::max(2, P.gx * elastic_window()) : remap3();
         dim3 grd(P.gx * P.gy * ((P.nx - H + P.kc - 1) / P.kc) + X.gather_blocks), blk(64, ty);
-        if (ty == 2) hipLaunchKernelGGL((vel3d_elastic_staged<O, 2>), grd, blk, 0, s, P, X);
-        else if (ty == 8) hipLaunchKernelGGL((vel3d_elastic_staged<O, 8>), grd, blk, 0, s, P, X);
-        else hipLaunchKernelGGL((vel3d_elastic_staged<O, 4>), grd, blk, 0, s, P, X);
+        if (ty == 2) hipLaunchKernelGGL((vel3d_elastic_staged<O, 2, RING>), grd, blk, 0, s, P, X);
+        else if (ty == 8) hipLaunchKernelGGL((vel3d_elastic_staged<O, 8, RING>), grd, blk, 0, s, P, X);
+        else hipLaunchKernelGGL((vel3d_elastic_staged<O, 4, RING>), grd, blk, 0, s, P, X);
         return;
     }
     const int kz = m.g.physics == 0 ? 1 : elastic_planes(ty);
@@ -1220,12 +1221,12 @@ void launch_vel3(const Model& m, hipStream_t s, VelParams3D P, const PassExtras&
     P.remap = m.g.physics == 0 && acoustic_window() ? std::max(2, P.gx * acoustic_window()) : remap3();
     P.xfast = m.g.physics == 1 && elastic_xfast();
     dim3 grd(P.gx * P.gy * ((P.nx - H + P.kc - 1) / P.kc) + X.gather_blocks), blk(64, ty, kz);
-    if (m.g.physics == 0 && nt_stores()) hipLaunchKernelGGL((vel3d_acoustic<O, true>), grd, blk, 0, s, P, X);
-    else if (m.g.physics == 0) hipLaunchKernelGGL((vel3d_acoustic<O, false>), grd, blk, 0, s, P, X);
-    else hipLaunchKernelGGL(vel3d_elastic<O>, grd, blk, 0, s, P, X);
+    if (m.g.physics == 0 && nt_stores()) hipLaunchKernelGGL((vel3d_acoustic<O, true, RING>), grd, blk, 0, s, P, X);
+    else if (m.g.physics == 0) hipLaunchKernelGGL((vel3d_acoustic<O, false, RING>), grd, blk, 0, s, P, X);
+    else hipLaunchKernelGGL((vel3d_elastic<O, RING>), grd, blk, 0, s, P, X);
 }
 
-template <int O>
+template <int O, bool RING>
 void launch_str3(const Model& m, hipStream_t s, StrParams3D P, const PassExtras& X)
 {
     P.gx = (P.nz + 63) / 64;
@@ -1236,13 +1237,13 @@ void launch_str3(const Model& m, hipStream_t s, StrParams3D P, const PassExtras&
         P.remap = elastic_window() ? std::max(2, P.gx * elastic_window()) : remap3();
         dim3 grd(P.gx * P.gy * ((P.nx + P.kc - 1) / P.kc) + X.gather_blocks), blk(64, ty);
         if (zstrip_prefetch(P.qz, P.npml, P.pml_mask)) {
-            if (ty == 2) hipLaunchKernelGGL((str3d_elastic_staged<O, 2, true>), grd, blk, 0, s, P, X);
-            else if (ty == 8) hipLaunchKernelGGL((str3d_elastic_staged<O, 8, true>), grd, blk, 0, s, P, X);
-            else hipLaunchKernelGGL((str3d_elastic_staged<O, 4, true>), grd, blk, 0, s, P, X);
+            if (ty == 2) hipLaunchKernelGGL((str3d_elastic_staged<O, 2, true, RING>), grd, blk, 0, s, P, X);
+            else if (ty == 8) hipLaunchKernelGGL((str3d_elastic_staged<O, 8, true, RING>), grd, blk, 0, s, P, X);
+            else hipLaunchKernelGGL((str3d_elastic_staged<O, 4, true, RING>), grd, blk, 0, s, P, X);
         } else {
-            if (ty == 2) hipLaunchKernelGGL((str3d_elastic_staged<O, 2, false>), grd, blk, 0, s, P, X);
-            else if (ty == 8) hipLaunchKernelGGL((str3d_elastic_staged<O, 8, false>), grd, blk, 0, s, P, X);
-            else hipLaunchKernelGGL((str3d_elastic_staged<O, 4, false>), grd, blk, 0, s, P, X);
+            if (ty == 2) hipLaunchKernelGGL((str3d_elastic_staged<O, 2, false, RING>), grd, blk, 0, s, P, X);
+            else if (ty == 8) hipLaunchKernelGGL((str3d_elastic_staged<O, 8, false, RING>), grd, blk, 0, s, P, X);
+            else hipLaunchKernelGGL((str3d_elastic_staged<O, 4, false, RING>), grd, blk, 0, s, P, X);
         }
         return;
     }
@@ -1251,9 +1252,9 @@ void launch_str3(const Model& m, hipStream_t s, StrParams3D P, const PassExtras&
     P.remap = m.g.physics == 0 && acoustic_window() ? std::max(2, P.gx * acoustic_window()) : remap3();
     P.xfast = m.g.physics == 1 && elastic_xfast();
     dim3 grd(P.gx * P.gy * ((P.nx + P.kc - 1) / P.kc) + X.gather_blocks), blk(64, ty, kz);
-    if (m.g.physics == 0 && nt_stores()) hipLaunchKernelGGL((str3d_acoustic<O, true>), grd, blk, 0, s, P, X);
-    else if (m.g.physics == 0) hipLaunchKernelGGL((str3d_acoustic<O, false>), grd, blk, 0, s, P, X);
-    else hipLaunchKernelGGL(str3d_elastic<O>, grd, blk, 0, s, P, X);
+    if (m.g.physics == 0 && nt_stores()) hipLaunchKernelGGL((str3d_acoustic<O, true, RING>), grd, blk, 0, s, P, X);
+    else if (m.g.physics == 0) hipLaunchKernelGGL((str3d_acoustic<O, false, RING>), grd, blk, 0, s, P, X);
+    else hipLaunchKernelGGL((str3d_elastic<O, RING>), grd, blk, 0, s, P, X);
 }
 
 }  // namespace
@@ -1315,6 +1316,7 @@ int velocity_pass_3d(const Model& m, const State& st, hipStream_t s, const PassE
     P.vx = st.field[GPI_VX];
     P.vy = st.field[GPI_VY];
     P.vz = st.field[GPI_VZ];
+    P.out = st.vout;
     P.cx = m.coef[GPI_C_DTINVAVXIRHO];   // acoustic pass
     P.cy = m.coef[GPI_C_DTINVAVYIRHO];
     P.cz = m.coef[GPI_C_DTINVAVZIRHO];
@@ -1335,10 +1337,10 @@ int velocity_pass_3d(const Model& m, const State& st, hipStream_t s, const PassE
     if (!state_complete(m, q, 9) || !P.vx || !P.vy || !P.vz || !P.s[0] || !P.rho || (ac && (!P.cx || !P.cy || !P.cz)))
         return -1;
     switch (m.g.order) {
-    case 2: launch_vel3<2>(m, s, P, X); break;
-    case 4: launch_vel3<4>(m, s, P, X); break;
-    case 6: launch_vel3<6>(m, s, P, X); break;
-    default: launch_vel3<8>(m, s, P, X); break;
+    case 2: P.out ? launch_vel3<2, true>(m, s, P, X) : launch_vel3<2, false>(m, s, P, X); break;
+    case 4: P.out ? launch_vel3<4, true>(m, s, P, X) : launch_vel3<4, false>(m, s, P, X); break;
+    case 6: P.out ? launch_vel3<6, true>(m, s, P, X) : launch_vel3<6, false>(m, s, P, X); break;
+    default: P.out ? launch_vel3<8, true>(m, s, P, X) : launch_vel3<8, false>(m, s, P, X); break;
     }
     return 0;
 }
@@ -1350,6 +1352,7 @@ int stress_pass_3d(const Model& m, const State& st, hipStream_t s, const PassExt
     P.vx = st.field[GPI_VX];
     P.vy = st.field[GPI_VY];
     P.vz = st.field[GPI_VZ];
+    P.out = st.sout;
     if (ac) {
         P.s[0] = st.field[GPI_P];
         P.c[0] = m.coef[GPI_C_DTK];
@@ -1386,10 +1389,10 @@ int stress_pass_3d(const Model& m, const State& st, hipStream_t s, const PassExt
     const Pml* q[9] = {&P.qx[0], &P.qx[1], &P.qx[2], &P.qy[0], &P.qy[1], &P.qy[2], &P.qz[0], &P.qz[1], &P.qz[2]};
     if (!state_complete(m, q, 9) || !P.vx || !P.vy || !P.vz || !P.s[0] || !P.c[0] || (!ac && !P.c[1])) return -1;
     switch (m.g.order) {
-    case 2: launch_str3<2>(m, s, P, X); break;
-    case 4: launch_str3<4>(m, s, P, X); break;
-    case 6: launch_str3<6>(m, s, P, X); break;
-    default: launch_str3<8>(m, s, P, X); break;
+    case 2: P.out ? launch_str3<2, true>(m, s, P, X) : launch_str3<2, false>(m, s, P, X); break;
+    case 4: P.out ? launch_str3<4, true>(m, s, P, X) : launch_str3<4, false>(m, s, P, X); break;
+    case 6: P.out ? launch_str3<6, true>(m, s, P, X) : launch_str3<6, false>(m, s, P, X); break;
+    default: P.out ? launch_str3<8, true>(m, s, P, X) : launch_str3<8, false>(m, s, P, X); break;
     }
     return 0;
 }

@@ -50,6 +50,8 @@ struct DevPoints {
 struct State {
     float* field[GPI_NFIELDS] = {};   // wavefields only (no derivative arrays)
     float* psi[GPI_NFIELDS] = {};     // CPML memory of derivative fields
+    // where a pass puts the velocities / stresses it updates, in floats behind those it reads
+    int64_t vout = 0, sout = 0;
     std::vector<void*> allocs;
     uint64_t bytes = 0;
 };
@@ -67,6 +69,15 @@ struct Model {
     State* st0 = nullptr;              // the state of gpi_forward / gpi_forward_save
     State* st1 = nullptr;              // 2-D: the state that several-step launches alternate with (made when first used)
     float* step_coef[5] = {};          // their coefficients (owned by st1)
+};
+
+// Wavefields that keep their last `slots` values: array f is base[f] with one slab per slot,
+// its current value in slot `cur`; arrays without a base are updated in place.
+struct Ring {
+    float* base[GPI_NFIELDS] = {};
+    int64_t slab = 0;
+    int slots = 1, cur = 0;
+    int after(int k) const { return (cur + k) % slots; }
 };
 
 struct Replay;
@@ -172,30 +183,34 @@ void negate_copy(float* dst, const float* src, int64_t n, hipStream_t s);
 // cur/prev/next: p1, vx1, vz1, p2, vx2, vz2 (pitched slabs); next <- cur after imaging
 void image_acoustic_2d(const Model& m, const float* const cur[6], const float* const prev[6], float* const next[6],
                        float* g_invK, float* g_rho, float dtI, hipStream_t s);
-// Imaging of one adjoint step with the exact forward wavefield (acoustic, 2-D and 3-D).
-// a2/c2/n2: the adjoint p and velocities (x, y, z; y unused in 2-D) before the step, after
-// it, and their copy destination; pa, pb: forward p_{n-1}, p_n; va, vb: forward v_n, v_{n+1}.
-// g_rho (and the velocity arguments) may be null.  Accumulators are FP64.
+// Imaging of consecutive adjoint steps with the exact forward wavefield (acoustic, 2-D and
+// 3-D).  a2: rings of the adjoint p and velocities (x, y, z; y unused in 2-D) whose slot
+// start + j holds the value before step j; pf, vf: forward p_{n-1} and v_n of the first step
+// (the next value one slab behind, the following steps' one slab before each).  pf with gK
+// or vf with g_rho may be null.  Accumulators are FP64.
 struct ImageSets {
     const float* a2[4];
-    const float* c2[4];
-    float* n2[4];
-    const float* pa;
-    const float* pb;
-    const float* va[3];
-    const float* vb[3];
+    int64_t slab;
+    int slots, start, steps;
+    const float* pf;
+    const float* vf[3];
 };
-// Elastic imaging of the checkpointed gradient (strips.hip).  Per forward step n: the
-// adjoint stresses before the adjoint stress pass (tau~^{n+1}), the adjoint velocities after
-// the adjoint velocity pass (v~^{n+1/2}) and the forward states around the step (tau^n,
-// tau^{n+1}, v^{n-1/2}, v^{n+1/2}).  Accumulated in FP64 on the slab layout:
+// Elastic imaging of the checkpointed gradient (strips.hip), `steps` consecutive adjoint
+// steps at once.  Per forward step n: the adjoint stresses before the adjoint stress pass
+// (tau~^{n+1}), the adjoint velocities after the adjoint velocity pass (v~^{n+1/2}) and the
+// forward states around the step (tau^n, tau^{n+1}, v^{n-1/2}, v^{n+1/2}).  The adjoint arrays
+// are rings: step j's stresses in slot start + j, its velocities in slot start + j + vshift;
+// the forward arrays f* point to the first step's earlier state, the later one is one slab
+// behind, the following steps' one slab before each.  Accumulated in FP64 on the slab layout:
 //   T = sum (tr tau~)(tr dtau) and P = sum tau~ . dtau over the normal stresses,
 //   S[s] = sum tau~_s dtau_s per shear stress, R[a] = sum v~_a dv_a per velocity.
 struct ElasticImage {
     int nn = 0, ns = 0, nv = 0;                     // normal, shear, velocity components
-    const float* an[3] = {}; const float* f0n[3] = {}; const float* f1n[3] = {};
-    const float* as[3] = {}; const float* f0s[3] = {}; const float* f1s[3] = {};
-    const float* av[3] = {}; const float* f0v[3] = {}; const float* f1v[3] = {};
+    int64_t slab = 0;
+    int slots = 1, start = 0, vshift = 0, steps = 0;
+    const float* an[3] = {}; const float* fn[3] = {};
+    const float* as[3] = {}; const float* fs[3] = {};
+    const float* av[3] = {}; const float* fv[3] = {};
     int shi[3][3] = {};                             // shear s occupies [0, shi) in (z, y, x)
     int sbase[3][3] = {};                           // its invmu average: cells p + sbase + {0, e1, e2, e1 + e2}
     int se1[3] = {}, se2[3] = {};                   // axes (0 z, 1 y, 2 x) of e1, e2
@@ -211,9 +226,9 @@ void image_elastic(const Model& m, const ElasticImage& E, hipStream_t s);
 void elastic_gradient(const Model& m, const ElasticImage& E, double* g_il, double* g_im, double* g_rho,
                       hipStream_t s);
 // Normal-stress sources inject dtM * a_n into every normal stress (src/fdtd/source.jl:79-119):
-// per target cell, acc += (sum of the adjoint normal stresses) * a_n at forward step n, and at
-// the end the part of the invlambda/invmu gradient that the Delta-tau form leaves out there.
-void source_trace(const DevPoints& pts, int64_t n, const float* const an[3], int nn, double* acc, hipStream_t s);
+// per target cell, acc += (sum of the adjoint normal stresses) * a_n at forward step n and the
+// E.steps - 1 steps before it, and at the end the part of the invlambda/invmu gradient that the Delta-tau form leaves out there.
+void source_trace(const DevPoints& pts, int64_t n, const ElasticImage& E, double* acc, hipStream_t s);
 void source_correction(const Model& m, const DevPoints& pts, const double* acc, int nn, double* g_il, double* g_im,
                        hipStream_t s);
 void image_acoustic_exact(const Model& m, const ImageSets& S, double* g_invK, double* g_rho, float dtI, hipStream_t s);

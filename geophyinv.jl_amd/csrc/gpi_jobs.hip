@@ -82,16 +82,23 @@ uint64_t job_bytes(const gpi_job& j)
     return b * 21 / 20 + (1 << 20);
 }
 
-// Device bytes a 2-D forward run takes on top when they are there (the state and coefficients
-// of the several-step launches; without them the passes run).
+// Device bytes a job takes on top when they are there: the state and coefficients of the
+// several-step launches (2-D; without them the passes run) and the adjoint arrays of the
+// steps imaged together (gradients; without them every step is imaged by itself).
 uint64_t job_optional_bytes(const gpi_job& j)
 {
     const gpi_grid& g = j.grid;
-    if (g.ndim != 2) return 0;
+    const bool d3 = g.ndim == 3, ac = g.physics == 0;
     const uint64_t h = (uint64_t)(g.order - 1), ld = (uint64_t)round_up(g.n[0] + (int64_t)h, 32);
-    const uint64_t slab = 4 * ld * ((uint64_t)g.n[2] + h);
-    const uint64_t face = std::max(ld, (uint64_t)g.n[2] + h), np = (uint64_t)std::max(g.npml, 0);
-    return (g.physics == 0 ? 5 * slab : 10 * slab) + (g.physics == 0 ? 4 : 8) * 2 * np * face * 4;
+    const uint64_t slab = 4 * ld * (uint64_t)(d3 ? g.n[1] + (int64_t)h : 1) * ((uint64_t)g.n[2] + h);
+    uint64_t b = 0;
+    if (!d3) {
+        const uint64_t face = std::max(ld, (uint64_t)g.n[2] + h), np = (uint64_t)std::max(g.npml, 0);
+        b = (ac ? 5 : 10) * slab + (ac ? 4 : 8) * 2 * np * face * 4;
+        if (j.checkpoint > 0) b *= 2;   // the adjoint wavefield's too
+    }
+    if (j.checkpoint > 0) b += 9 * (ac ? (d3 ? 4 : 3) : (d3 ? 9 : 5)) * slab;
+    return b;
 }
 
 int run_job(gpi_ctx* c, const gpi_job& j)

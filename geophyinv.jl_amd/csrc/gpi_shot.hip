@@ -614,6 +614,180 @@ int run_shot(gpi_ctx* c, Model& m, const gpi_shot* shot, Store* save)
     return GPI_OK;
 }
 
+// Wavefield w of a checkpointed gradient: its arrays with a ring move through the ring's
+// slots (the passes write the next slot, so keeping the history costs no copies), the
+// others stay in the state.  2-D shots advance several steps per launch where they can.
+struct Mover {
+    gpi_ctx* c;
+    const Model& m;
+    State w;                 // field pointers at the current slot
+    Ring ring;
+    const Sources& src;
+    PassExtras XV, XS;
+    StepPlan plan;
+    bool stepped = false;
+    int64_t* launches;
+
+    // current slot 0, as the state that a checkpoint is restored into
+    void rewind()
+    {
+        ring.cur = 0;
+        plan.cur = 0;
+        at_slot();
+    }
+    void at_slot()
+    {
+        for (int f = 0; f < GPI_NFIELDS; ++f)
+            if (ring.base[f]) w.field[f] = ring.base[f] + ring.slab * ring.cur;
+    }
+    // the velocities of step it (in the next slot on return)
+    int velocities(int64_t it)
+    {
+        XV.it = XS.it = it;
+        const int64_t d = ring.slab * (ring.after(1) - ring.cur);
+        w.vout = ring.base[GPI_VX] ? d : 0;
+        const int rc = velocity_pass(c, m, w, XV);
+        if (rc) return rc;
+        for (int f : {GPI_VX, GPI_VY, GPI_VZ})
+            if (ring.base[f]) w.field[f] += d;
+        for (int q : src.vfall) inject(m, w, src.pts[q], it, c->stream);
+        *launches += 1 + (int64_t)src.vfall.size();
+        return GPI_OK;
+    }
+    // its stresses: the ring moves on
+    int stresses(int64_t it)
+    {
+        const int64_t d = ring.slab * (ring.after(1) - ring.cur);
+        w.sout = ring.base[m.g.physics == 0 ? GPI_P : GPI_TAUXX] ? d : 0;
+        const int rc = stress_pass(c, m, w, XS);
+        if (rc) return rc;
+        ring.cur = ring.after(1);
+        at_slot();
+        for (int q : src.sfall) inject(m, w, src.pts[q], it, c->stream);
+        *launches += 1 + (int64_t)src.sfall.size();
+        return GPI_OK;
+    }
+    // n steps from it
+    int advance(int64_t it, int64_t n)
+    {
+        while (n > 0) {
+            const int k = stepped ? (int)std::min<int64_t>(n, plan.steps) : 1;
+            if (stepped) {
+                run_steps_2d(m, plan, it, k, c->stream, &ring);
+                *launches += plan.launches;
+            } else {
+                const int rc = velocities(it);
+                if (rc) return rc;
+                if (const int rs = stresses(it)) return rs;
+            }
+            it += k;
+            n -= k;
+        }
+        return GPI_OK;
+    }
+};
+
+// Slabs of a ring, every cell zero: the passes leave the cells outside their ranges alone.
+int alloc_ring(gpi_ctx* c, Scratch& S, const Model& m, Ring& r, const std::vector<int>& fields, int slots)
+{
+    r.slab = m.slab;
+    r.slots = slots;
+    for (int f : fields) {
+        const int rc = S.alloc(&r.base[f], (size_t)slots * (size_t)m.slab);
+        if (rc) return rc;
+    }
+    for (int f : fields)
+        HIPTRY(c, hipMemsetAsync(r.base[f], 0, sizeof(float) * (size_t)slots * (size_t)m.slab, c->stream));
+    return GPI_OK;
+}
+
+// The adjoint wavefield's arrays over up to IMAGE_STEPS steps, which one imaging launch then
+// reads together; fewer where memory is short, down to the arrays themselves (imaged between
+// the two passes of every step) where `inplace_ok`.
+constexpr int IMAGE_STEPS = 8;
+
+struct AdjointRing {
+    gpi_ctx* c;
+    Ring ring;
+    State st, alt;           // memory variables and the arrays outside the ring; alt: for plan_mover
+    Scratch* S = nullptr;
+    explicit AdjointRing(gpi_ctx* cc) : c(cc) {}
+    ~AdjointRing() { drop(); }
+    AdjointRing(const AdjointRing&) = delete;
+    AdjointRing& operator=(const AdjointRing&) = delete;
+    void drop()
+    {
+        (void)hipStreamSynchronize(c->stream);
+        delete S;
+        S = nullptr;
+        free_allocs(c, st.allocs, st.bytes);
+        free_allocs(c, alt.allocs, alt.bytes);
+        st = State{};
+        alt = State{};
+        ring = Ring{};
+    }
+    bool inplace() const { return ring.slots == 1; }
+    int steps() const { return std::max(1, ring.slots - 1); }
+    int take(const Model& m, const std::vector<int>& fields, bool inplace_ok)
+    {
+        int rc = GPI_ENOMEM;
+        for (int n = IMAGE_STEPS; n >= (inplace_ok ? 0 : 1) && rc == GPI_ENOMEM; n /= 2) {
+            drop();
+            S = new Scratch(c);
+            rc = alloc_ring(c, *S, m, ring, fields, n + 1);
+            if (!rc) rc = alloc_state(c, m, &st, true, &ring);
+            if (rc == GPI_ENOMEM) (void)hipGetLastError();
+            if (n == 0) break;
+        }
+        return rc;
+    }
+};
+
+// Several steps per launch for a 2-D mover; `adj`: the adjoint wavefield (its second state is
+// its own, the forward one's the model's).
+int plan_mover(Mover& M, Scratch& S, int64_t nt, AdjointRing* adj)
+{
+    gpi_ctx* c = M.c;
+    if (M.m.g.ndim != 2 || (adj && adj->inplace())) return GPI_OK;
+    int rc = plan_steps_2d(c, const_cast<Model&>(M.m), S, nt, M.src, nullptr, {}, &M.plan, &M.stepped);
+    if (rc || !M.stepped) return rc;
+    if (adj) {
+        if ((rc = alloc_state(c, M.m, &adj->alt, true, &adj->ring))) {
+            if (rc != GPI_ENOMEM) return rc;
+            (void)hipGetLastError();
+            M.stepped = false;
+            return GPI_OK;
+        }
+        M.plan.st[0] = &adj->st;
+        M.plan.st[1] = &adj->alt;
+    }
+    return GPI_OK;
+}
+
+// cnt <= A.steps() adjoint steps from `it` of mover B and their imaging
+template <typename Image>
+int adjoint_steps(Mover& B, const AdjointRing& A, Sampler& smp, int64_t it, int64_t cnt, Image&& image)
+{
+    gpi_ctx* c = B.c;
+    int rc;
+    if (B.stepped) {
+        if ((rc = B.advance(it, cnt))) return rc;
+        return image();
+    }
+    for (int64_t j = 0; j < cnt; ++j) {
+        hipEvent_t* E = smp.at(it + j);
+        if (E) HIPTRY(c, hipEventRecord(E[0], c->stream));
+        if ((rc = B.velocities(it + j))) return rc;
+        if (E) HIPTRY(c, hipEventRecord(E[1], c->stream));
+        if (A.inplace() && (rc = image())) return rc;
+        if (E) HIPTRY(c, hipEventRecord(E[2], c->stream));
+        if ((rc = B.stresses(it + j))) return rc;
+        if (E) HIPTRY(c, hipEventRecord(E[3], c->stream));
+        smp.done(it + j);
+    }
+    return A.inplace() ? GPI_OK : image();
+}
+
 int check_shot(gpi_ctx* c, uint64_t model, const gpi_shot* shot, Model** out)
 {
     if (!c || !shot) return fail(c, GPI_EINVAL, "null argument");
@@ -810,128 +984,91 @@ int gpi_adjoint_checkpoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi
     if (!(dtI > 0.0f) || !std::isfinite(dtI)) return fail(c, GPI_EINVAL, "dtI must be positive");
     HIPTRY(c, hipSetDevice(c->device));
     const bool rho = g_rho != nullptr;
-    const State& s1 = *m.st0;
     Scratch S(c);
-    struct Held {
-        gpi_ctx* c;
-        State st;
-        ~Held()
-        {
-            (void)hipStreamSynchronize(c->stream);
-            free_allocs(c, st.allocs, st.bytes);
-        }
-    } h2{c, State{}};
-    int rc = alloc_state(c, m, &h2.st, true);
-    if (rc) return rc;
-    const State& s2 = h2.st;
+    int rc;
     PassExtras XV2{}, XS2{};
     Sources src2;
     if ((rc = plan_sources(c, m, S, shot->nsrc2, shot->src2, shot->wav2, nt, true, XV2, XS2, src2))) return rc;
-    PassExtras XV1 = R.xv, XS1 = R.xs;
 
     // velocity components present: x, (y,) z
     std::vector<int> vf;
     for (int f : {GPI_VX, GPI_VY, GPI_VZ})
         if (field_codes(g.ndim, g.physics, f)) vf.push_back(f);
-    const int nv = (int)vf.size();
     const int64_t C = sv.every;
     const int64_t K = (nt + C - 1) / C;
     const int64_t L = std::min(C, nt);
     const size_t slab = (size_t)m.slab;
     const size_t bytes = sizeof(float) * slab;
-    // segment buffers: p_{n0-1} .. p_{n1-1} and (for rho) v_{n0} .. v_{n1}
-    float* segP = nullptr;
-    float* segV[3] = {};
-    float* vnext[3] = {};
-    if ((rc = S.alloc(&segP, (size_t)(L + 1) * slab))) return rc;
+    int64_t launches = 0;
+    // the segment's forward wavefield: p_{n0-1} .. p_{n1-1} in slots 0 .. L and, for rho, v_{n0-1}
+    // .. v_{n1} in slots 0 .. L + 1, the last one from the segment after it
+    Mover F{c, m, *m.st0, {}, R.src, R.xv, R.xs, {}, false, &launches};
+    if ((rc = alloc_ring(c, S, m, F.ring, {GPI_P}, (int)(L + 1)))) return rc;
+    if (rho && (rc = alloc_ring(c, S, m, F.ring, vf, (int)(L + 2)))) return rc;
+    float* vnext[GPI_NFIELDS] = {};
     if (rho)
-        for (int d = 0; d < nv; ++d)
-            if ((rc = S.alloc(&segV[d], (size_t)(L + 1) * slab)) || (rc = S.alloc(&vnext[d], slab))) return rc;
-    // adjoint velocities before the step (for rho), two alternating sets; the adjoint p
-    // before the step is the one the stress pass starts from (the velocity pass leaves p),
-    // so the imaging reads it there and keeps no copy
-    float* tp[2][4] = {};
-    if (rho)
-        for (auto& set : tp)
-            for (int d = 0; d < nv; ++d)
-                if ((rc = S.alloc(&set[1 + d], slab))) return rc;
+        for (int f : vf)
+            if ((rc = S.alloc(&vnext[f], slab))) return rc;
     double *gK = nullptr, *gR = nullptr;
     if ((rc = S.alloc(&gK, slab))) return rc;
     if (rho && (rc = S.alloc(&gR, slab))) return rc;
+    // the adjoint wavefield: p before and (for rho) v around up to IMAGE_STEPS steps
+    AdjointRing A(c);
+    std::vector<int> kept{GPI_P};
+    if (rho) kept.insert(kept.end(), vf.begin(), vf.end());
+    if ((rc = A.take(m, kept, !rho))) return rc;
+    Mover B{c, m, A.st, A.ring, src2, XV2, XS2, {}, false, &launches};
+    if (c->sample_ev.empty()) {
+        if ((rc = plan_mover(F, S, nt, nullptr)) || (rc = plan_mover(B, *A.S, nt, &A))) return rc;
+    }
     HIPTRY(c, hipMemsetAsync(gK, 0, sizeof(double) * slab, c->stream));
     if (rho) HIPTRY(c, hipMemsetAsync(gR, 0, sizeof(double) * slab, c->stream));
-    if ((rc = zero_state(c, m, s2, c->stream))) return rc;
-    for (auto& set : tp)
-        for (float* p : set)
-            if (p) HIPTRY(c, hipMemsetAsync(p, 0, bytes, c->stream));
+    B.rewind();
+    if ((rc = zero_state(c, m, B.w, c->stream))) return rc;
     if (rho)   // v_nt: the trailing half step of the stored run
-        for (int d = 0; d < nv; ++d)
-            HIPTRY(c, hipMemcpyAsync(vnext[d], sv.snap[vf[d]], bytes, hipMemcpyDeviceToDevice, c->stream));
+        for (int f : vf) HIPTRY(c, hipMemcpyAsync(vnext[f], sv.snap[f], bytes, hipMemcpyDeviceToDevice, c->stream));
 
     Sampler smp(c, nt);
-    int64_t launches = 0, it = 0;
+    int64_t it = 0;
     HIPTRY(c, hipEventRecord(c->ev[0], c->stream));
     for (int64_t k = K - 1; k >= 0; --k) {
         const int64_t n0 = k * C, n1 = std::min(n0 + C, nt);
         // the forward state before step n0, then the segment recomputed with its sources
-        if (k == 0) rc = zero_state(c, m, s1, c->stream);
-        else rc = copy_state(c, m, s1, sv.ckpt[k - 1], false, c->stream);
-        if (rc) return rc;
-        HIPTRY(c, hipMemcpyAsync(segP, s1.field[GPI_P], bytes, hipMemcpyDeviceToDevice, c->stream));
-        for (int64_t n = n0; n < n1; ++n) {
-            XV1.it = XS1.it = n;
-            if ((rc = velocity_pass(c, m, s1, XV1))) return rc;
-            for (int q : R.src.vfall) inject(m, s1, R.src.pts[q], n, c->stream);
-            if ((rc = stress_pass(c, m, s1, XS1))) return rc;
-            for (int q : R.src.sfall) inject(m, s1, R.src.pts[q], n, c->stream);
-            HIPTRY(c, hipMemcpyAsync(segP + (size_t)(n - n0 + 1) * slab, s1.field[GPI_P], bytes,
-                                     hipMemcpyDeviceToDevice, c->stream));
-            if (rho)
-                for (int d = 0; d < nv; ++d)
-                    HIPTRY(c, hipMemcpyAsync(segV[d] + (size_t)(n - n0) * slab, s1.field[vf[d]], bytes,
-                                             hipMemcpyDeviceToDevice, c->stream));
-            launches += 2 + (int64_t)(R.src.vfall.size() + R.src.sfall.size());
-        }
+        F.rewind();
+        if (k == 0) rc = zero_state(c, m, F.w, c->stream);
+        else rc = copy_state(c, m, F.w, sv.ckpt[k - 1], false, c->stream);
+        if (rc || (rc = F.advance(n0, n1 - n0))) return rc;
         if (rho)
-            for (int d = 0; d < nv; ++d)
-                HIPTRY(c, hipMemcpyAsync(segV[d] + (size_t)(n1 - n0) * slab, vnext[d], bytes,
+            for (int f : vf)
+                HIPTRY(c, hipMemcpyAsync(F.ring.base[f] + (size_t)(n1 - n0 + 1) * slab, vnext[f], bytes,
                                          hipMemcpyDeviceToDevice, c->stream));
-        // the adjoint steps of this segment, forward step n = nt - 1 - it
-        for (int64_t n = n1 - 1; n >= n0; --n, ++it) {
-            hipEvent_t* E = smp.at(it);
-            XV2.it = XS2.it = it;
-            if (E) HIPTRY(c, hipEventRecord(E[0], c->stream));
-            if ((rc = velocity_pass(c, m, s2, XV2))) return rc;
-            if (E) HIPTRY(c, hipEventRecord(E[1], c->stream));
-            for (int q : src2.vfall) inject(m, s2, src2.pts[q], it, c->stream);
+        // the adjoint steps of this segment, forward step n = nt - 1 - it, and their imaging
+        for (int64_t n = n1 - 1; n >= n0;) {
+            const int64_t cnt = std::min<int64_t>(A.steps(), n - n0 + 1);
             ImageSets I{};
-            float* const* prev = tp[it & 1];
-            float* const* next = tp[(it + 1) & 1];
-            I.a2[0] = s2.field[GPI_P];                   // p2 before the step
-            I.pa = segP + (size_t)(n - n0) * slab;       // p_{n-1}
-            I.pb = segP + (size_t)(n - n0 + 1) * slab;   // p_n
-            image_acoustic_exact(m, I, gK, nullptr, dtI, c->stream);   // invK term
-            if (E) HIPTRY(c, hipEventRecord(E[2], c->stream));
-            if ((rc = stress_pass(c, m, s2, XS2))) return rc;
-            if (E) HIPTRY(c, hipEventRecord(E[3], c->stream));
-            if (rho) {   // density term: v2 before the step (a copy), then keep this step's v2
-                ImageSets Iv{};
-                for (int d = 0; d < nv; ++d) {
-                    const int a = vf[d] - GPI_VX;   // 0 x, 1 y, 2 z
-                    Iv.a2[1 + a] = prev[1 + d];
-                    Iv.c2[1 + a] = s2.field[vf[d]];
-                    Iv.n2[1 + a] = next[1 + d];
-                    Iv.va[a] = segV[d] + (size_t)(n - n0) * slab;       // v_n
-                    Iv.vb[a] = segV[d] + (size_t)(n - n0 + 1) * slab;   // v_{n+1}
+            I.slab = m.slab;
+            I.slots = B.ring.slots;
+            I.start = B.ring.cur;
+            I.steps = (int)cnt;
+            I.a2[0] = B.ring.base[GPI_P];
+            I.pf = F.ring.base[GPI_P] + (size_t)(n - n0) * slab;   // p_{n-1}
+            if (rho)
+                for (int f : vf) {
+                    I.a2[1 + f - GPI_VX] = B.ring.base[f];
+                    I.vf[f - GPI_VX] = F.ring.base[f] + (size_t)(n - n0 + 1) * slab;   // v_n
                 }
-                image_acoustic_exact(m, Iv, nullptr, gR, dtI, c->stream);
-            }
-            launches += (rho ? 4 : 3) + (int64_t)src2.vfall.size();
-            smp.done(it);
+            auto image = [&] {
+                image_acoustic_exact(m, I, gK, gR, dtI, c->stream);
+                ++launches;
+                return GPI_OK;
+            };
+            if ((rc = adjoint_steps(B, A, smp, it, cnt, image))) return rc;
+            it += cnt;
+            n -= cnt;
         }
         if (rho)
-            for (int d = 0; d < nv; ++d)
-                HIPTRY(c, hipMemcpyAsync(vnext[d], segV[d], bytes, hipMemcpyDeviceToDevice, c->stream));
+            for (int f : vf)
+                HIPTRY(c, hipMemcpyAsync(vnext[f], F.ring.base[f] + slab, bytes, hipMemcpyDeviceToDevice, c->stream));
     }
     if ((rc = finish_timing(c, smp, nt, launches))) return rc;
     int64_t n3[3];
@@ -966,24 +1103,11 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
     HIPTRY(c, hipSetDevice(c->device));
     const bool d3 = g.ndim == 3;
     const int H = m.h;
-    const State& s1 = *m.st0;
     Scratch S(c);
-    struct Held {
-        gpi_ctx* c;
-        State st;
-        ~Held()
-        {
-            (void)hipStreamSynchronize(c->stream);
-            free_allocs(c, st.allocs, st.bytes);
-        }
-    } h2{c, State{}};
-    int rc = alloc_state(c, m, &h2.st, true);
-    if (rc) return rc;
-    const State& s2 = h2.st;
+    int rc;
     PassExtras XV2{}, XS2{};
     Sources src2;
     if ((rc = plan_sources(c, m, S, shot->nsrc2, shot->src2, shot->wav2, nt, true, XV2, XS2, src2))) return rc;
-    PassExtras XV1 = R.xv, XS1 = R.xs;
 
     // components, their regions on the slab (z, y, x) and their coefficient stencils
     const int nz = (int)g.n[0], ny = d3 ? (int)g.n[1] : 1, nx = (int)g.n[2];
@@ -1029,14 +1153,13 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
     const int64_t C = sv.every;
     const int64_t L = std::min(C, nt);
     const size_t slab = (size_t)m.slab;
-    const size_t bytes = sizeof(float) * slab;
-    // segment buffers: the forward stresses tau^{n0} .. tau^{n1} and velocities v^{n0-1/2} .. v^{n1-1/2}
+    // the segment's forward wavefield: tau^{n0} .. tau^{n1} and v^{n0-1/2} .. v^{n1-1/2} in slots 0 .. L
     std::vector<int> all = nf;
     all.insert(all.end(), sf.begin(), sf.end());
     all.insert(all.end(), vf.begin(), vf.end());
-    std::vector<float*> seg(all.size(), nullptr);
-    for (float*& p : seg)
-        if ((rc = S.alloc(&p, (size_t)(L + 1) * slab))) return rc;
+    int64_t launches = 0;
+    Mover F{c, m, *m.st0, {}, R.src, R.xv, R.xs, {}, false, &launches};
+    if ((rc = alloc_ring(c, S, m, F.ring, all, (int)(L + 1)))) return rc;
     double* acc[8] = {};
     const int nacc = 2 + E.ns + E.nv;
     for (int q = 0; q < nacc; ++q) {
@@ -1047,7 +1170,15 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
     E.P = acc[1];
     for (int q = 0; q < E.ns; ++q) E.S[q] = acc[2 + q];
     for (int q = 0; q < E.nv; ++q) E.R[q] = acc[2 + E.ns + q];
-    if ((rc = zero_state(c, m, s2, c->stream))) return rc;
+    // the adjoint wavefield: its arrays around up to IMAGE_STEPS steps
+    AdjointRing A(c);
+    if ((rc = A.take(m, all, true))) return rc;
+    Mover B{c, m, A.st, A.ring, src2, XV2, XS2, {}, false, &launches};
+    if (c->sample_ev.empty()) {
+        if ((rc = plan_mover(F, S, nt, nullptr)) || (rc = plan_mover(B, *A.S, nt, &A))) return rc;
+    }
+    B.rewind();
+    if ((rc = zero_state(c, m, B.w, c->stream))) return rc;
     // normal-stress sources of the forward run: their per-target traces (source_trace)
     std::vector<int> nsrc;
     std::vector<double*> sacc;
@@ -1060,64 +1191,41 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
         nsrc.push_back((int)q);
         sacc.push_back(a);
     }
-    auto save = [&](int64_t slot) -> int {
-        for (size_t q = 0; q < all.size(); ++q)
-            HIPTRY(c, hipMemcpyAsync(seg[q] + (size_t)slot * slab, s1.field[all[q]], bytes, hipMemcpyDeviceToDevice,
-                                     c->stream));
-        return GPI_OK;
-    };
+    E.slab = m.slab;
+    E.slots = B.ring.slots;
+    E.vshift = A.inplace() ? 0 : 1;
+    for (int q = 0; q < E.nn; ++q) E.an[q] = B.ring.base[nf[q]];
+    for (int q = 0; q < E.ns; ++q) E.as[q] = B.ring.base[sf[q]];
+    for (int q = 0; q < E.nv; ++q) E.av[q] = B.ring.base[vf[q]];
 
     Sampler smp(c, nt);
-    int64_t launches = 0, it = 0;
+    int64_t it = 0;
     const int64_t K = (nt + C - 1) / C;
     HIPTRY(c, hipEventRecord(c->ev[0], c->stream));
     for (int64_t k = K - 1; k >= 0; --k) {
         const int64_t n0 = k * C, n1 = std::min(n0 + C, nt);
-        if (k == 0) rc = zero_state(c, m, s1, c->stream);
-        else rc = copy_state(c, m, s1, sv.ckpt[k - 1], false, c->stream);
-        if (rc || (rc = save(0))) return rc;
-        for (int64_t n = n0; n < n1; ++n) {
-            XV1.it = XS1.it = n;
-            if ((rc = velocity_pass(c, m, s1, XV1))) return rc;
-            for (int q : R.src.vfall) inject(m, s1, R.src.pts[q], n, c->stream);
-            if ((rc = stress_pass(c, m, s1, XS1))) return rc;
-            for (int q : R.src.sfall) inject(m, s1, R.src.pts[q], n, c->stream);
-            if ((rc = save(n - n0 + 1))) return rc;
-            launches += 2 + (int64_t)(R.src.vfall.size() + R.src.sfall.size());
-        }
-        // adjoint steps of this segment (forward step n = nt - 1 - it), imaging between the passes
-        for (int64_t n = n1 - 1; n >= n0; --n, ++it) {
-            hipEvent_t* Ev = smp.at(it);
-            XV2.it = XS2.it = it;
-            if (Ev) HIPTRY(c, hipEventRecord(Ev[0], c->stream));
-            if ((rc = velocity_pass(c, m, s2, XV2))) return rc;
-            if (Ev) HIPTRY(c, hipEventRecord(Ev[1], c->stream));
-            for (int q : src2.vfall) inject(m, s2, src2.pts[q], it, c->stream);
-            const size_t a = (size_t)(n - n0) * slab, b = a + slab;
-            int w = 0;
-            for (int q = 0; q < E.nn; ++q, ++w) {
-                E.an[q] = s2.field[nf[q]];
-                E.f0n[q] = seg[w] + a;
-                E.f1n[q] = seg[w] + b;
-            }
-            for (int q = 0; q < E.ns; ++q, ++w) {
-                E.as[q] = s2.field[sf[q]];
-                E.f0s[q] = seg[w] + a;
-                E.f1s[q] = seg[w] + b;
-            }
-            for (int q = 0; q < E.nv; ++q, ++w) {
-                E.av[q] = s2.field[vf[q]];
-                E.f0v[q] = seg[w] + a;
-                E.f1v[q] = seg[w] + b;
-            }
-            image_elastic(m, E, c->stream);
-            for (size_t q = 0; q < nsrc.size(); ++q) source_trace(R.src.pts[nsrc[q]], n, E.an, E.nn, sacc[q], c->stream);
-            if (Ev) HIPTRY(c, hipEventRecord(Ev[2], c->stream));
-            if ((rc = stress_pass(c, m, s2, XS2))) return rc;
-            for (int q : src2.sfall) inject(m, s2, src2.pts[q], it, c->stream);
-            if (Ev) HIPTRY(c, hipEventRecord(Ev[3], c->stream));
-            launches += 3 + (int64_t)(src2.vfall.size() + src2.sfall.size());
-            smp.done(it);
+        F.rewind();
+        if (k == 0) rc = zero_state(c, m, F.w, c->stream);
+        else rc = copy_state(c, m, F.w, sv.ckpt[k - 1], false, c->stream);
+        if (rc || (rc = F.advance(n0, n1 - n0))) return rc;
+        // adjoint steps of this segment (forward step n = nt - 1 - it) and their imaging
+        for (int64_t n = n1 - 1; n >= n0;) {
+            const int64_t cnt = std::min<int64_t>(A.steps(), n - n0 + 1);
+            const size_t f = (size_t)(n - n0) * slab;
+            for (int q = 0; q < E.nn; ++q) E.fn[q] = F.ring.base[nf[q]] + f;
+            for (int q = 0; q < E.ns; ++q) E.fs[q] = F.ring.base[sf[q]] + f;
+            for (int q = 0; q < E.nv; ++q) E.fv[q] = F.ring.base[vf[q]] + f;
+            E.start = B.ring.cur;
+            E.steps = (int)cnt;
+            auto image = [&] {
+                image_elastic(m, E, c->stream);
+                for (size_t q = 0; q < nsrc.size(); ++q) source_trace(R.src.pts[nsrc[q]], n, E, sacc[q], c->stream);
+                ++launches;
+                return GPI_OK;
+            };
+            if ((rc = adjoint_steps(B, A, smp, it, cnt, image))) return rc;
+            it += cnt;
+            n -= cnt;
         }
     }
     if ((rc = finish_timing(c, smp, nt, launches))) return rc;

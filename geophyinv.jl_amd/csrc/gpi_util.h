@@ -53,7 +53,8 @@ void free_model(gpi_ctx* c, Model* m);
 int alloc_coef(gpi_ctx* c, Model& m, int id);
 
 // wavefields + CPML memory of one propagating wavefield of model m
-int alloc_state(gpi_ctx* c, const Model& m, State* st, bool reuse = false);
+// skip: without the arrays of this ring
+int alloc_state(gpi_ctx* c, const Model& m, State* st, bool reuse = false, const Ring* skip = nullptr);
 void free_state(gpi_ctx* c, State* st);
 int zero_state(gpi_ctx* c, const Model& m, const State& st, hipStream_t s);
 size_t psi_floats(const Model& m, int f);

@@ -278,10 +278,10 @@ size_t psi_floats(const Model& m, int f)
     return ax == 2 ? (size_t)(P.ps2 * 2 * m.g.npml) : (size_t)(P.ps2 * n3[2]);
 }
 
-int alloc_state(gpi_ctx* c, const Model& m, State* st, bool reuse)
+int alloc_state(gpi_ctx* c, const Model& m, State* st, bool reuse, const Ring* skip)
 {
     for (int f = GPI_P; f <= GPI_TAUYZ; ++f) {
-        if (!field_codes(m.g.ndim, m.g.physics, f)) continue;
+        if (!field_codes(m.g.ndim, m.g.physics, f) || (skip && skip->base[f])) continue;
         int rc = dev_alloc(c, &st->allocs, &st->bytes, (void**)&st->field[f], sizeof(float) * (size_t)m.slab,
                            reuse);
         if (rc) return rc;

@@ -96,11 +96,13 @@ __global__ __launch_bounds__(256) void image2d_kernel(ImageParams P)
     for (int k = 0; k < 6; ++k) P.next[k][o] = P.cur[k][o];
 }
 
-// Imaging with the exact forward wavefield, one thread per cell of the pitched slab
-// (z rows to the pitch, y columns to the y pitch, x to nx + h): the copy of the adjoint
-// fields into the next set covers every field's extent, the gradients their own ranges.
-// Each step's term is formed in FP32 with the reference's expressions and added to the
-// FP64 accumulators.
+// Imaging with the exact forward wavefield, one thread per cell of the pitched slab (z rows
+// to the pitch, y columns to the y pitch, x to nx + h), over consecutive steps: each step's
+// term is formed in FP32 with the reference's expressions and added to the FP64 accumulators
+// in step order.  Memory-bound: a step reads the adjoint and the forward value once (8 bytes
+// per cell for invK; a forward value serves two steps), and the accumulators move once per
+// launch, against 28 bytes a step (and the copy of p into its history, 8 more) when every
+// step was imaged by itself.
 struct ImageExactParams {
     ImageSets S;
     double* gK;
@@ -126,30 +128,50 @@ __global__ __launch_bounds__(256) void image_exact_kernel(ImageExactParams P)
     const ImageSets& S = P.S;
     if (P.gK && i < P.nz && j < P.ny && k < P.nx) {
         // compute_gmodKI!: p2_prev * (p1_prev - p1) * dtI, p1 = -p_forward
-        const float t = (S.a2[0][o] * (S.pa[o] - S.pb[o])) * P.dtI;
-        P.gK[o] = P.gK[o] + (double)t;
+        const float* f = S.pf + o;
+        float pb = f[S.slab];
+        double g = P.gK[o];
+        int slot = S.start;
+        for (int n = 0; n < S.steps; ++n, f -= S.slab) {
+            const float pa = *f;
+            const float t = (S.a2[0][o + S.slab * slot] * (pa - pb)) * P.dtI;
+            g = g + (double)t;
+            pb = pa;
+            if (++slot == S.slots) slot = 0;
+        }
+        P.gK[o] = g;
     }
     const int h = P.h;
     if (P.gR && i < P.nz - 2 * h && k < P.nx - 2 * h && (P.ndim == 2 || j < P.ny - 2 * h)) {
         // compute_gmodrho! buffers at the two samples of each @av_*i, then combine_gmodrho!
         const int jh = P.ndim == 2 ? 0 : j + h;
-        auto buf = [&](int a, int64_t q) { return (S.a2[1 + a][q] * (S.va[a][q] - S.vb[a][q])) * P.dtI; };
-        const int64_t ax = (i + h) + sy * jh + sx * k;     // @av_xi: x pair
-        const int64_t az = i + sy * jh + sx * (k + h);     // @av_zi: z pair
-        const float avx = (buf(0, ax) + buf(0, ax + sx)) * 0.5f;
-        const float avz = (buf(2, az) + buf(2, az + 1)) * 0.5f;
+        const int64_t ax = (i + h) + sy * jh + sx * k;        // @av_xi: x pair
+        const int64_t az = i + sy * jh + sx * (k + h);        // @av_zi: z pair
+        const int64_t ay = (i + h) + sy * j + sx * (k + h);   // @av_yi: y pair
         const int64_t g = (i + h) + sy * jh + sx * (k + h);
-        double r = P.gR[g] - (double)avx;
-        if (P.ndim == 3) {
-            const int64_t ay = (i + h) + sy * j + sx * (k + h);   // @av_yi: y pair
-            r = r - (double)((buf(1, ay) + buf(1, ay + sy)) * 0.5f);
+        const int64_t q[6] = {ax, ax + sx, ay, ay + sy, az, az + 1};
+        float vb[6];
+#pragma unroll
+        for (int e = 0; e < 6; ++e)
+            if (P.ndim == 3 || e < 2 || e > 3) vb[e] = S.vf[e / 2][q[e] + S.slab];
+        double r = P.gR[g];
+        int slot = S.start;
+        for (int n = 0; n < S.steps; ++n) {
+            float buf[6];
+#pragma unroll
+            for (int e = 0; e < 6; ++e) {
+                if (P.ndim == 2 && (e == 2 || e == 3)) continue;
+                const float va = S.vf[e / 2][q[e] - S.slab * n];
+                buf[e] = (S.a2[1 + e / 2][q[e] + S.slab * slot] * (va - vb[e])) * P.dtI;
+                vb[e] = va;
+            }
+            r = r - (double)((buf[0] + buf[1]) * 0.5f);
+            if (P.ndim == 3) r = r - (double)((buf[2] + buf[3]) * 0.5f);
+            r = r - (double)((buf[4] + buf[5]) * 0.5f);
+            if (++slot == S.slots) slot = 0;
         }
-        P.gR[g] = r - (double)avz;
+        P.gR[g] = r;
     }
-    if (S.n2[0]) S.n2[0][o] = S.c2[0][o];
-    if (P.gR)
-        for (int a = 0; a < 3; ++a)
-            if (S.n2[1 + a]) S.n2[1 + a][o] = S.c2[1 + a][o];
 }
 
 // ---- elastic imaging ----------------------------------------------------------------
@@ -189,6 +211,11 @@ __device__ __forceinline__ void slab_coords(int64_t o, int ld, int py, int c[3])
     c[2] = (int)(r / py);
 }
 
+// One thread per cell over E.steps consecutive steps: every adjoint and forward value is
+// read once per step (a forward value serves two) and the accumulators once per launch; 72
+// bytes per cell and step in 3-D (2-D 40) and 128 / steps for the accumulators, against 236
+// (140) when every step was imaged by itself, and no copies into the histories (72 and 40).
+template <int NN, int NS, int NV>
 __global__ __launch_bounds__(256) void image_elastic_kernel(ElasticParams P)
 {
     const int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -196,25 +223,76 @@ __global__ __launch_bounds__(256) void image_elastic_kernel(ElasticParams P)
     int c[3];
     slab_coords(o, P.ld, P.py, c);
     const ElasticImage& E = P.E;
-    if (c[0] < P.nz && c[1] < P.ny && c[2] < P.nx) {
-        double ta = 0.0, td = 0.0, dot = 0.0;
-        for (int q = 0; q < E.nn; ++q) {
-            const double t = (double)E.an[q][o];
-            const double d = (double)E.f1n[q][o] - (double)E.f0n[q][o];
-            ta += t;
-            td += d;
-            dot += t * d;
-        }
-        E.T[o] += ta * td;
-        E.P[o] += dot;
+    const bool un = c[0] < P.nz && c[1] < P.ny && c[2] < P.nx;
+    bool us[NS], uv[NV];
+    float n1[NN], s1[NS], v1[NV];
+    double T = 0.0, D = 0.0, Ss[NS], R[NV];
+    if (un) {
+        T = E.T[o];
+        D = E.P[o];
+#pragma unroll
+        for (int q = 0; q < NN; ++q) n1[q] = E.fn[q][o + E.slab];
     }
-    for (int q = 0; q < E.ns; ++q)
-        if (c[0] < E.shi[q][0] && c[1] < E.shi[q][1] && c[2] < E.shi[q][2])
-            E.S[q][o] += (double)E.as[q][o] * ((double)E.f1s[q][o] - (double)E.f0s[q][o]);
-    for (int q = 0; q < E.nv; ++q)
-        if (c[0] >= E.vlo[q][0] && c[0] < E.vhi[q][0] && c[1] >= E.vlo[q][1] && c[1] < E.vhi[q][1] &&
-            c[2] >= E.vlo[q][2] && c[2] < E.vhi[q][2])
-            E.R[q][o] += (double)E.av[q][o] * ((double)E.f1v[q][o] - (double)E.f0v[q][o]);
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        us[q] = c[0] < E.shi[q][0] && c[1] < E.shi[q][1] && c[2] < E.shi[q][2];
+        if (us[q]) {
+            Ss[q] = E.S[q][o];
+            s1[q] = E.fs[q][o + E.slab];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        uv[q] = c[0] >= E.vlo[q][0] && c[0] < E.vhi[q][0] && c[1] >= E.vlo[q][1] && c[1] < E.vhi[q][1] &&
+                c[2] >= E.vlo[q][2] && c[2] < E.vhi[q][2];
+        if (uv[q]) {
+            R[q] = E.R[q][o];
+            v1[q] = E.fv[q][o + E.slab];
+        }
+    }
+    for (int n = 0; n < E.steps; ++n) {
+        const int64_t f = o - E.slab * n;
+        const int64_t a = o + E.slab * ((E.start + n) % E.slots), av = o + E.slab * ((E.start + n + E.vshift) % E.slots);
+        if (un) {
+            double ta = 0.0, td = 0.0, dot = 0.0;
+#pragma unroll
+            for (int q = 0; q < NN; ++q) {
+                const float n0 = E.fn[q][f];
+                const double t = (double)E.an[q][a];
+                const double d = (double)n1[q] - (double)n0;
+                n1[q] = n0;
+                ta += t;
+                td += d;
+                dot += t * d;
+            }
+            T += ta * td;
+            D += dot;
+        }
+#pragma unroll
+        for (int q = 0; q < NS; ++q)
+            if (us[q]) {
+                const float s0 = E.fs[q][f];
+                Ss[q] += (double)E.as[q][a] * ((double)s1[q] - (double)s0);
+                s1[q] = s0;
+            }
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+            if (uv[q]) {
+                const float v0 = E.fv[q][f];
+                R[q] += (double)E.av[q][av] * ((double)v1[q] - (double)v0);
+                v1[q] = v0;
+            }
+    }
+    if (un) {
+        E.T[o] = T;
+        E.P[o] = D;
+    }
+#pragma unroll
+    for (int q = 0; q < NS; ++q)
+        if (us[q]) E.S[q][o] = Ss[q];
+#pragma unroll
+    for (int q = 0; q < NV; ++q)
+        if (uv[q]) E.R[q][o] = R[q];
 }
 
 __global__ __launch_bounds__(256) void elastic_gradient_kernel(ElasticParams P, const float* __restrict__ il,
@@ -264,23 +342,28 @@ __global__ __launch_bounds__(256) void elastic_gradient_kernel(ElasticParams P, 
     gr[o] = r / (2.0 * dt);
 }
 
-// The normal-stress source of forward step n at each target: a_n = sum of weight x wavelet
-// (the injection sum of the stress pass), times the trace of the adjoint normal stresses.
+// The normal-stress source of forward steps n, n - 1, .. at each target: a_n = sum of weight x
+// wavelet (the injection sum of the stress pass), times the trace of the adjoint normal
+// stresses.
 __global__ __launch_bounds__(256) void source_trace_kernel(const int64_t* __restrict__ toff,
                                                            const int32_t* __restrict__ tptr,
                                                            const int32_t* __restrict__ tsrc,
                                                            const float* __restrict__ tw, const float* __restrict__ wav,
-                                                           int npts, int ntarget, int64_t n, const float* t0,
-                                                           const float* t1, const float* t2, double* acc)
+                                                           int npts, int ntarget, int64_t n, ElasticImage E,
+                                                           double* acc)
 {
     const int t = (int)(blockIdx.x * 256 + threadIdx.x);
     if (t >= ntarget) return;
-    float a = 0.0f;
-    for (int k = tptr[t]; k < tptr[t + 1]; ++k) a = a + tw[k] * wav[n * npts + tsrc[k]];
-    const int64_t c = toff[t];
-    double tr = (double)t0[c] + (double)t1[c];
-    if (t2) tr += (double)t2[c];
-    acc[t] += tr * (double)a;
+    double sum = acc[t];
+    for (int j = 0; j < E.steps; ++j) {
+        float a = 0.0f;
+        for (int k = tptr[t]; k < tptr[t + 1]; ++k) a = a + tw[k] * wav[(n - j) * npts + tsrc[k]];
+        const int64_t c = toff[t] + E.slab * ((E.start + j) % E.slots);
+        double tr = (double)E.an[0][c] + (double)E.an[1][c];
+        if (E.nn == 3) tr += (double)E.an[2][c];
+        sum += tr * (double)a;
+    }
+    acc[t] = sum;
 }
 
 // With a = M + (d-1)L the trace eigenvalue of the normal block and Q = acc (adjoint run
@@ -321,7 +404,9 @@ ElasticParams elastic_params(const Model& m, const ElasticImage& E)
 void image_elastic(const Model& m, const ElasticImage& E, hipStream_t s)
 {
     const ElasticParams P = elastic_params(m, E);
-    hipLaunchKernelGGL(image_elastic_kernel, dim3((unsigned)((P.slab + 255) / 256)), dim3(256), 0, s, P);
+    const dim3 grd((unsigned)((P.slab + 255) / 256)), blk(256);
+    if (m.g.ndim == 3) hipLaunchKernelGGL((image_elastic_kernel<3, 3, 3>), grd, blk, 0, s, P);
+    else hipLaunchKernelGGL((image_elastic_kernel<2, 1, 2>), grd, blk, 0, s, P);
 }
 
 void elastic_gradient(const Model& m, const ElasticImage& E, double* g_il, double* g_im, double* g_rho,
@@ -333,13 +418,12 @@ void elastic_gradient(const Model& m, const ElasticImage& E, double* g_il, doubl
                        g_il, g_im, g_rho);
 }
 
-void source_trace(const DevPoints& pts, int64_t n, const float* const an[3], int nn, double* acc, hipStream_t s)
+void source_trace(const DevPoints& pts, int64_t n, const ElasticImage& E, double* acc, hipStream_t s)
 {
     if (pts.ntarget <= 0) return;
     hipLaunchKernelGGL(source_trace_kernel, dim3((unsigned)((pts.ntarget + 255) / 256)), dim3(256), 0, s,
                        (const int64_t*)pts.toff, (const int32_t*)pts.tptr, (const int32_t*)pts.tsrc,
-                       (const float*)pts.tw, (const float*)pts.wav, pts.npts, pts.ntarget, n, an[0], an[1],
-                       nn > 2 ? an[2] : (const float*)nullptr, acc);
+                       (const float*)pts.tw, (const float*)pts.wav, pts.npts, pts.ntarget, n, E, acc);
 }
 
 void source_correction(const Model& m, const DevPoints& pts, const double* acc, int nn, double* g_il, double* g_im,
