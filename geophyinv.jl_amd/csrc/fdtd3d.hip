@@ -234,7 +234,9 @@ __global__ __launch_bounds__(512) void vel3d_acoustic(VelParams3D P, PassExtras 
         L.czo = bload(plane_rsrc(P.cz, s2, k, np), lc);
     };
     auto update = [&](int k, const Ops& cur) {
-        const int bt = bx + P.gx * (by + P.gy * k);
+        const VelParams3D& Q = fresh(P);
+        const PassExtras& Y = fresh(P, X);
+        const int bt = bx + Q.gx * (by + Q.gy * k);
         const int iu = opaque(i), ju = opaque(j);
         const int o = (iu + H) + s1 * (ju + H) + s2 * (k + H);   // @inn of every velocity
         // vx on (nz-2h, ny-2h, nx-h): dpdx = D_xi(p)
@@ -242,36 +244,36 @@ __global__ __launch_bounds__(512) void vel3d_acoustic(VelParams3D P, PassExtras 
 #pragma unroll
             for (int m = 0; m < O - 1; ++m) w[m] = w[m + 1];
             w[O - 1] = cur.wn;
-            float d = stencil<O>(w) * P.dxI;
-            d = cpml3_x<false>(d, P.qx[0], iu, ju, k, P.npml, P.pml_mask);
+            float d = stencil<O>(w) * Q.dxI;
+            d = cpml3_x<false>(d, Q.qx[0], iu, ju, k, Q.npml, Q.pml_mask);
             float nv = cur.vxo + cur.cxo * d;
-            if ((P.rigid_mask & GPI_FACE(2, 0)) && k == 0) into<RING>(P.vx, P.out)[(iu + H) + s1 * (ju + H)] = -nv;
-            if ((P.rigid_mask & GPI_FACE(2, 1)) && k == P.nx - H - 1)
-                into<RING>(P.vx, P.out)[(iu + H) + s1 * (ju + H) + s2 * (P.nx + H - 1)] = -nv;
-            if (X.ninj) nv = inject_velocity(X, INJ_VX, bt, o, nv, P.rho, P.dt);
-            store_out<NT>(&into<RING>(P.vx, P.out)[o], nv);
+            if ((Q.rigid_mask & GPI_FACE(2, 0)) && k == 0) into<RING>(Q.vx, Q.out)[(iu + H) + s1 * (ju + H)] = -nv;
+            if ((Q.rigid_mask & GPI_FACE(2, 1)) && k == Q.nx - H - 1)
+                into<RING>(Q.vx, Q.out)[(iu + H) + s1 * (ju + H) + s2 * (Q.nx + H - 1)] = -nv;
+            if (Y.ninj) nv = inject_velocity(Y, INJ_VX, bt, o, nv, Q.rho, Q.dt);
+            store_out<NT>(&into<RING>(Q.vx, Q.out)[o], nv);
         }
         // vy on (nz-2h, ny-h, nx-2h): dpdy = D_yi(p)
-        if (ycol && k < P.nx - 2 * H) {
-            float d = stencil<O>(cur.py) * P.dyI;
-            d = cpml3_y<false>(d, P.qy[0], iu, ju, k, P.npml, P.pml_mask);
+        if (ycol && k < Q.nx - 2 * H) {
+            float d = stencil<O>(cur.py) * Q.dyI;
+            d = cpml3_y<false>(d, Q.qy[0], iu, ju, k, Q.npml, Q.pml_mask);
             float nv = cur.vyo + cur.cyo * d;
-            if ((P.rigid_mask & GPI_FACE(1, 0)) && ju == 0) into<RING>(P.vy, P.out)[(iu + H) + s2 * (k + H)] = -nv;
-            if ((P.rigid_mask & GPI_FACE(1, 1)) && ju == P.ny - H - 1)
-                into<RING>(P.vy, P.out)[(iu + H) + s1 * (P.ny + H - 1) + s2 * (k + H)] = -nv;
-            if (X.ninj) nv = inject_velocity(X, INJ_VY, bt, o, nv, P.rho, P.dt);
-            store_out<NT>(&into<RING>(P.vy, P.out)[o], nv);
+            if ((Q.rigid_mask & GPI_FACE(1, 0)) && ju == 0) into<RING>(Q.vy, Q.out)[(iu + H) + s2 * (k + H)] = -nv;
+            if ((Q.rigid_mask & GPI_FACE(1, 1)) && ju == Q.ny - H - 1)
+                into<RING>(Q.vy, Q.out)[(iu + H) + s1 * (Q.ny + H - 1) + s2 * (k + H)] = -nv;
+            if (Y.ninj) nv = inject_velocity(Y, INJ_VY, bt, o, nv, Q.rho, Q.dt);
+            store_out<NT>(&into<RING>(Q.vy, Q.out)[o], nv);
         }
         // vz on (nz-h, ny-2h, nx-2h): dpdz = D_zi(p)
-        if (zcol && k < P.nx - 2 * H) {
-            float d = stencil<O>(cur.pz) * P.dzI;
-            d = cpml3_z<false>(d, P.qz[0], iu, ju, k, P.npml, P.pml_mask);
+        if (zcol && k < Q.nx - 2 * H) {
+            float d = stencil<O>(cur.pz) * Q.dzI;
+            d = cpml3_z<false>(d, Q.qz[0], iu, ju, k, Q.npml, Q.pml_mask);
             float nv = cur.vzo + cur.czo * d;
-            if ((P.rigid_mask & GPI_FACE(0, 0)) && iu == 0) into<RING>(P.vz, P.out)[s1 * (ju + H) + s2 * (k + H)] = -nv;
-            if ((P.rigid_mask & GPI_FACE(0, 1)) && iu == P.nz - H - 1)
-                into<RING>(P.vz, P.out)[(P.nz + H - 1) + s1 * (ju + H) + s2 * (k + H)] = -nv;
-            if (X.ninj) nv = inject_velocity(X, INJ_VZ, bt, o, nv, P.rho, P.dt);
-            store_out<NT>(&into<RING>(P.vz, P.out)[o], nv);
+            if ((Q.rigid_mask & GPI_FACE(0, 0)) && iu == 0) into<RING>(Q.vz, Q.out)[s1 * (ju + H) + s2 * (k + H)] = -nv;
+            if ((Q.rigid_mask & GPI_FACE(0, 1)) && iu == Q.nz - H - 1)
+                into<RING>(Q.vz, Q.out)[(Q.nz + H - 1) + s1 * (ju + H) + s2 * (k + H)] = -nv;
+            if (Y.ninj) nv = inject_velocity(Y, INJ_VZ, bt, o, nv, Q.rho, Q.dt);
+            store_out<NT>(&into<RING>(Q.vz, Q.out)[o], nv);
         }
     };
     // two planes per trip with alternating operand sets: no register whose load may be
@@ -919,7 +921,8 @@ __global__ __launch_bounds__(64 * TY) void vel3d_elastic_staged(VelParams3D P, P
             v.e3 = lds_z<O, W>(Lzz, ty + H, tx) * P.dzI;   // D_zi(tauzz) at (i, j+h, k+h)
             const int bt = bx + P.gx * (by + P.gy * k);
             const int io = opaque(i), jo = __builtin_amdgcn_readfirstlane(opaque(j));
-            vel3d_elastic_update<O, RING>(P, X, io, jo, k, bt, (io + H) + s1 * (jo + H) + s2 * p, ux, uy, uz, v);
+            vel3d_elastic_update<O, RING>(fresh(P), fresh(P, X), io, jo, k, bt, (io + H) + s1 * (jo + H) + s2 * p, ux,
+                                          uy, uz, v);
         }
         if (p < plast) {   // plane p+1 (loaded) into the other slot; loads for the next planes
 #pragma unroll
@@ -930,6 +933,11 @@ __global__ __launch_bounds__(64 * TY) void vel3d_elastic_staged(VelParams3D P, P
     }
 }
 
+// (both passes: the update reads its parameters anew each plane, fresh(): 359 against 340 us
+// a step on 190 x 201 x 210, 180 against 162 on 140 x 136 x 151, 1644 against 1598 on 360^3;
+// taken there for the z-strips too, the stress pass ran 3 % slower.  Loading the x and y
+// strips' memory variables a plane ahead like the z-strips', in registers freed by a third
+// staging slot, ran 14 - 25 % slower: more loads and scalar work on every plane.)
 // order 2: six waves per SIMD (80 registers; 81 in the ring form without the bound)
 template <int O, int TY, bool ZP, bool RING>
 __global__ __launch_bounds__(64 * TY, (O == 2 ? 6 : 1)) void str3d_elastic_staged(StrParams3D P, PassExtras X)
@@ -1055,7 +1063,8 @@ __global__ __launch_bounds__(64 * TY, (O == 2 ? 6 : 1)) void str3d_elastic_stage
                 v.xza = zstrip_apply(v.xza, zm[1], Lz, 1, P.qz[1], io, jo, k, P.npml, P.pml_mask, uxz);
                 v.yza = zstrip_apply(v.yza, zm[2], Lz, 2, P.qz[2], io, jo, k, P.npml, P.pml_mask, uyz);
             }
-            str3d_elastic_update<O, RING, ZP>(P, X, io, jo, k, bt, io + s1 * jo + s2 * k, un, uxz, uxy, uyz, v);
+            str3d_elastic_update<O, RING, ZP>(fresh(P), fresh(P, X), io, jo, k, bt, io + s1 * jo + s2 * k, un, uxz, uxy, uyz,
+                                              v);
         }
         if (p < plast) {   // plane p+1 (loaded) into the other slot; loads for the next planes
 #pragma unroll

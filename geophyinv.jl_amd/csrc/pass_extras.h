@@ -26,6 +26,39 @@ __device__ __forceinline__ float* into(float* p, int64_t out)
     return RING ? p + out : p;
 }
 
+struct PassExtras;
+
+// A kernel's argument block (the argument `local`, `offset` bytes into the block) read anew
+// from here on: its fields are scalar loads where they are used instead of values that the
+// compiler loads before a loop and, once the scalar registers are full, keeps in lanes of
+// vector registers (a third of the vector instructions of the 3-D passes were such moves).
+template <typename T>
+__device__ __forceinline__ const T& fresh_arg(const T& local, int offset)
+{
+#if defined(__AMDGCN__)
+    (void)local;
+    const __attribute__((address_space(4))) char* k =
+        (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    return *(const T*)(k + offset);
+#else
+    (void)offset;
+    return local;
+#endif
+}
+
+// the two arguments (parameters, extras) of a pass
+template <typename T>
+__device__ __forceinline__ const T& fresh(const T& P)
+{
+    return fresh_arg(P, 0);
+}
+template <typename T>
+__device__ __forceinline__ const PassExtras& fresh(const T&, const PassExtras& X)
+{
+    return fresh_arg(X, (int)((sizeof(T) + 7) / 8 * 8));
+}
+
 enum InjKind { INJ_P = 0, INJ_NORMAL2 = 1, INJ_NORMAL3 = 2, INJ_VX = 3, INJ_VY = 4, INJ_VZ = 5 };
 
 // Workgroup order for the 8 XCDs of MI355X: workgroups are dispatched to XCDs round
