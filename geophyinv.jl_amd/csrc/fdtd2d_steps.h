@@ -57,6 +57,13 @@ struct StepParams2D {
     float* hist[5];
     int64_t hslab;
     int hslots, hstart;
+    // time reversal (acoustic): before every step p takes stored values on three planes inside
+    // the absorbing strips at both ends of each axis (boundary_force!); fx: nt x 6 columns of
+    // nz, fz: nt x nx columns of 6, read at fnt - 1 - it; fnp the strips' width per axis (z, x)
+    const float* fx;
+    const float* fz;
+    int64_t fnt;
+    int fnp[2];
     int ntile;
     const TileBox* box;
     int64_t it0;

@@ -103,8 +103,9 @@ struct TileLds {
 // coefficient is zero, so only the stores of tiles on the grid's edge are masked.
 // SR: the tile may hold sources and receivers.  KEEP: every step is kept (a ring).  Both cost
 // the inner tiles registers, and with them the second tile per CU (KEEP: 21.1 against 15.3 ms
-// for 800 steps of 2-D elastic 2081^2), so they are choices at compile time.
-template <int O, int PHYS, int RZ, int WX, int NT, bool PX, bool PZ, bool SR, bool KEEP>
+// for 800 steps of 2-D elastic 2081^2), so they are choices at compile time.  FORCE:
+// time reversal, p forced on stored planes before every step.
+template <int O, int PHYS, int RZ, int WX, int NT, bool PX, bool PZ, bool SR, bool KEEP, bool FORCE>
 __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q, const TileBox& B)
 {
     using T = Tile<O, PHYS, RZ, WX, NT>;
@@ -134,6 +135,28 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
         for (int f = 0; f < NF; ++f) S[k][f] = in ? at(P.in[f], o) : 0.0f;
 #pragma unroll
         for (int f = 0; f < NF; ++f) C[k][f] = in ? at(P.coef[f], o) : 0.0f;
+    }
+    // stored planes: this thread's offset in one step's values of fx (>= 0) or fz (~offset), or none
+    constexpr int NONE = INT32_MIN;
+    int foff[FORCE ? K : 1];
+    auto forced = [&](int k, int64_t it) __attribute__((always_inline)) {
+        const int64_t n = P.fnt - 1 - it;
+        const int o = foff[FORCE ? k : 0];
+        return o >= 0 ? P.fx[n * (6 * (int64_t)P.nz) + o] : P.fz[n * (6 * (int64_t)P.nx) + ~o];
+    };
+    if constexpr (FORCE) {
+        auto plane = [](int p, int n, int np) { return p >= np && p < np + 3 ? p - np : p >= n - np - 3 && p < n - np ? p - (n - np) + 6 : -1; };
+        const int az = r >= 0 && r < P.nz ? plane(r, P.nz, P.fnp[0]) : -1;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int c = cc + k;
+            foff[k] = NONE;
+            if (r < 0 || r >= P.nz || c < 0 || c >= P.nx) continue;
+            const int ax = plane(c, P.nx, P.fnp[1]);
+            if (ax >= 0) foff[k] = r + P.nz * ax;
+            else if (az >= 0) foff[k] = ~(az + 6 * c);
+            if (foff[k] != NONE) S[k][0] = forced(k, P.it0);
+        }
     }
     float px[K][PX ? ND : 1], pz[K][PZ ? ND : 1], za[ND], zb[ND], zk[ND], xa[K][ND], xb[K][ND], xk[K][ND];
     int zi[ND];
@@ -254,6 +277,7 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
         for (int k = 0; k < K; ++k) {
             const int c = cc + k;
             if (!own || c < cxl || c >= cxh) continue;
+            if (FORCE && f0 == 0 && (r >= P.nz || c >= P.nx)) continue;   // not yet restored there
 #pragma unroll
             for (int f = 0; f < NF; ++f)
                 if (f >= f0 && f < f1 && P.hist[f]) at(P.hist[f] + P.hslab * slot, r + ld * c) = S[k][f];
@@ -265,6 +289,12 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
         const int64_t it = P.it0 + s;
         float anext = 0.0f;
         if (SR && tid < ns && s + 1 < P.steps) anext = *(amp_next += P.namp);
+        float fnext[FORCE ? K : 1];
+        if constexpr (FORCE) {
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (s + 1 < P.steps && foff[k] != NONE) fnext[k] = forced(k, it + 1);
+        }
         const float* amp = Q.amp + (s & 1) * MAX_TILE_SOURCES;
         // columns whose values are still needed: the rest of the halo is stale already
         const int need0 = P.lead - (P.steps - 1 - s) * H;
@@ -277,7 +307,7 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
 #pragma unroll
                     for (int f = 0; f < FVX; ++f) S[k][f] = L[RZ * k + f * A];
             }
-            if (KEEP && s) keep(0, FVX, s);
+            if (KEEP && !FORCE && s) keep(0, FVX, s);
 #pragma unroll
             for (int k = 0; k < K; ++k) {
                 const float* l = L + RZ * k;
@@ -404,6 +434,12 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
                     }
                 }
             }
+            if constexpr (FORCE) {   // kept as the step left it, and forced for the next one
+                if (s + 1 < P.steps) keep(0, FVX, s + 1);
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if (s + 1 < P.steps && foff[k] != NONE) S[k][0] = fnext[k];
+            }
 #pragma unroll
             for (int k = 0; k < K; ++k) {
                 float* l = L + RZ * k;
@@ -454,7 +490,7 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
     }
 }
 
-template <int O, int PHYS, int RZ, int WX, int NT, bool KEEP>
+template <int O, int PHYS, int RZ, int WX, int NT, bool KEEP, bool FORCE>
 __global__ __launch_bounds__(NT) void steps2d_kernel(StepParams2D P)
 {
     using T = Tile<O, PHYS, RZ, WX, NT>;
@@ -469,21 +505,21 @@ __global__ __launch_bounds__(NT) void steps2d_kernel(StepParams2D P)
     const int r0 = B.z0 - P.lead, c0 = B.x0 - P.lead, e = H + P.npml + 1;
     const bool pz = r0 < e || r0 + RZ > P.nz - H - e, px = c0 < e || c0 + WX > P.nx - H - e;
     if (px) {
-        if (pz) run_tile<O, PHYS, RZ, WX, NT, true, true, true, KEEP>(P, Q, B);
-        else run_tile<O, PHYS, RZ, WX, NT, true, false, true, KEEP>(P, Q, B);
+        if (pz) run_tile<O, PHYS, RZ, WX, NT, true, true, true, KEEP, FORCE>(P, Q, B);
+        else run_tile<O, PHYS, RZ, WX, NT, true, false, true, KEEP, FORCE>(P, Q, B);
     } else {
-        if (pz) run_tile<O, PHYS, RZ, WX, NT, false, true, true, KEEP>(P, Q, B);
-        else run_tile<O, PHYS, RZ, WX, NT, false, false, true, KEEP>(P, Q, B);
+        if (pz) run_tile<O, PHYS, RZ, WX, NT, false, true, true, KEEP, FORCE>(P, Q, B);
+        else run_tile<O, PHYS, RZ, WX, NT, false, false, true, KEEP, FORCE>(P, Q, B);
     }
 }
 
 // Tiles away from the strips and faces, without sources and receivers.
-template <int O, int PHYS, int RZ, int WX, int NT, bool KEEP>
+template <int O, int PHYS, int RZ, int WX, int NT, bool KEEP, bool FORCE>
 __global__ __launch_bounds__(NT) void steps2d_inner_kernel(StepParams2D P)
 {
     using T = Tile<O, PHYS, RZ, WX, NT>;
     __shared__ float f[T::FLOATS];
-    run_tile<O, PHYS, RZ, WX, NT, false, false, false, KEEP>(P, TileLds{f, nullptr, nullptr, nullptr},
+    run_tile<O, PHYS, RZ, WX, NT, false, false, false, KEEP, FORCE>(P, TileLds{f, nullptr, nullptr, nullptr},
                                                        P.box[xcd_remap(blockIdx.x, gridDim.x)]);
 }
 
@@ -546,15 +582,29 @@ struct Region {
 template <int O, int PHYS, int RZ, int WX, int NT>
 void launch_all(const StepParams2D& P, hipStream_t s)
 {
-    if (P.hslots) hipLaunchKernelGGL((steps2d_kernel<O, PHYS, RZ, WX, NT, true>), dim3(P.ntile), dim3(NT), 0, s, P);
-    else hipLaunchKernelGGL((steps2d_kernel<O, PHYS, RZ, WX, NT, false>), dim3(P.ntile), dim3(NT), 0, s, P);
+    const dim3 grd(P.ntile), blk(NT);
+    if constexpr (PHYS == 0) {
+        if (P.fx) {
+            hipLaunchKernelGGL((steps2d_kernel<O, PHYS, RZ, WX, NT, true, true>), grd, blk, 0, s, P);
+            return;
+        }
+    }
+    if (P.hslots) hipLaunchKernelGGL((steps2d_kernel<O, PHYS, RZ, WX, NT, true, false>), grd, blk, 0, s, P);
+    else hipLaunchKernelGGL((steps2d_kernel<O, PHYS, RZ, WX, NT, false, false>), grd, blk, 0, s, P);
 }
 
 template <int O, int PHYS, int RZ, int WX, int NT>
 void launch_inner(const StepParams2D& P, hipStream_t s)
 {
-    if (P.hslots) hipLaunchKernelGGL((steps2d_inner_kernel<O, PHYS, RZ, WX, NT, true>), dim3(P.ntile), dim3(NT), 0, s, P);
-    else hipLaunchKernelGGL((steps2d_inner_kernel<O, PHYS, RZ, WX, NT, false>), dim3(P.ntile), dim3(NT), 0, s, P);
+    const dim3 grd(P.ntile), blk(NT);
+    if constexpr (PHYS == 0) {
+        if (P.fx) {
+            hipLaunchKernelGGL((steps2d_inner_kernel<O, PHYS, RZ, WX, NT, true, true>), grd, blk, 0, s, P);
+            return;
+        }
+    }
+    if (P.hslots) hipLaunchKernelGGL((steps2d_inner_kernel<O, PHYS, RZ, WX, NT, true, false>), grd, blk, 0, s, P);
+    else hipLaunchKernelGGL((steps2d_inner_kernel<O, PHYS, RZ, WX, NT, false, false>), grd, blk, 0, s, P);
 }
 
 // The tiles that pick_tiles chooses from.

@@ -437,6 +437,20 @@ int copy_records(gpi_ctx* c, const std::vector<DevPoints>& rec, int64_t nt, floa
     return GPI_OK;
 }
 
+// Slabs of a ring, every cell zero: the passes leave the cells outside their ranges alone.
+int alloc_ring(gpi_ctx* c, Scratch& S, const Model& m, Ring& r, const std::vector<int>& fields, int slots)
+{
+    r.slab = m.slab;
+    r.slots = slots;
+    for (int f : fields) {
+        const int rc = S.alloc(&r.base[f], (size_t)slots * (size_t)m.slab);
+        if (rc) return rc;
+    }
+    for (int f : fields)
+        HIPTRY(c, hipMemsetAsync(r.base[f], 0, sizeof(float) * (size_t)slots * (size_t)m.slab, c->stream));
+    return GPI_OK;
+}
+
 // mod_x_proc! for one supersource in :forward (save == nullptr) or :forward_save mode
 // (src/fdtd/propagate.jl:138-261).
 int run_shot(gpi_ctx* c, Model& m, const gpi_shot* shot, Store* save)
@@ -508,8 +522,21 @@ int run_shot(gpi_ctx* c, Model& m, const gpi_shot* shot, Store* save)
     // several steps per launch where nothing is taken from the wavefield between the steps
     StepPlan plan;
     bool stepped = false;
-    if (g.ndim == 2 && !illum && !(save && !ckpt) && c->sample_ev.empty())
+    if (g.ndim == 2 && !illum && c->sample_ev.empty())
         if ((rc = plan_steps_2d(c, m, S, nt, src, shot, rec, &plan, &stepped))) return rc;
+    // boundary saving keeps every step of the stored fields of one launch in a ring
+    Ring kept;
+    if (stepped && save && !ckpt) {
+        std::vector<int> fields(save->field, save->field + save->nfield);
+        rc = alloc_ring(c, S, m, kept, fields, plan.steps + 1);
+        if (rc == GPI_ENOMEM) {
+            (void)hipGetLastError();
+            kept = Ring{};
+            stepped = false;
+        } else if (rc) {
+            return rc;
+        }
+    }
     // the launches of a shot end at checkpoints and snapshots
     auto launch_steps = [&](int64_t it) {
         int64_t n = std::min<int64_t>(plan.steps, nt - it);
@@ -534,10 +561,28 @@ int run_shot(gpi_ctx* c, Model& m, const gpi_shot* shot, Store* save)
     HIPTRY(c, hipEventRecord(c->ev[0], c->stream));
     for (int64_t it = 0; stepped && it < nt;) {
         const int n = launch_steps(it);
-        run_steps_2d(m, plan, it, n, c->stream);
+        const bool strips = save && !ckpt;
+        const int first = kept.after(1);
+        run_steps_2d(m, plan, it, n, c->stream, strips ? &kept : nullptr);
         launches += plan.launches;
+        for (int q = 0; strips && q < save->nfield; ++q) {
+            int64_t fn[3];
+            shape_of(g.ndim, g.order, g.physics, g.n, save->field[q], fn);
+            for (int ax = 2; ax >= 0; ax -= 2) {
+                strip_ring(m, kept, save->field[q], fn, ax, strip_np(m, ax), first, n,
+                           save->strip[q][ax] + save->strip_size[q][ax] * it, c->stream);
+                ++launches;
+            }
+        }
         it += n;
-        const State& now = *plan.st[plan.cur];
+        State now = *plan.st[plan.cur];
+        for (int f = 0; strips && f < GPI_NFIELDS; ++f)
+            if (kept.base[f]) {
+                now.field[f] = kept.base[f] + kept.slab * kept.cur;
+                if (it == nt)
+                    HIPTRY(c, hipMemcpyAsync(st.field[f], now.field[f], sizeof(float) * (size_t)m.slab,
+                                             hipMemcpyDeviceToDevice, c->stream));
+            }
         if (ckpt && it % save->every == 0 && it / save->every <= (int64_t)save->ckpt.size())
             if ((rc = copy_state(c, m, now, save->ckpt[it / save->every - 1], true, c->stream))) return rc;
         for (int q = 0; q < shot->nsnap; ++q)
@@ -686,20 +731,6 @@ struct Mover {
         return GPI_OK;
     }
 };
-
-// Slabs of a ring, every cell zero: the passes leave the cells outside their ranges alone.
-int alloc_ring(gpi_ctx* c, Scratch& S, const Model& m, Ring& r, const std::vector<int>& fields, int slots)
-{
-    r.slab = m.slab;
-    r.slots = slots;
-    for (int f : fields) {
-        const int rc = S.alloc(&r.base[f], (size_t)slots * (size_t)m.slab);
-        if (rc) return rc;
-    }
-    for (int f : fields)
-        HIPTRY(c, hipMemsetAsync(r.base[f], 0, sizeof(float) * (size_t)slots * (size_t)m.slab, c->stream));
-    return GPI_OK;
-}
 
 // The adjoint wavefield's arrays over up to IMAGE_STEPS steps, which one imaging launch then
 // reads together; fewer where memory is short, down to the arrays themselves (imaged between
@@ -873,6 +904,64 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
     HIPTRY(c, hipSetDevice(c->device));
     const State& s1 = *m.st0;
     Scratch S(c);
+    int rc;
+    PassExtras XV1{}, XS1{}, XV2{}, XS2{};
+    Sources src1, src2;
+    if ((rc = plan_sources(c, m, S, shot->nsrc1, shot->src1, shot->wav1, nt, false, XV1, XS1, src1))) return rc;
+    if ((rc = plan_sources(c, m, S, shot->nsrc2, shot->src2, shot->wav2, nt, true, XV2, XS2, src2))) return rc;
+    float *gK, *gR;
+    if ((rc = S.alloc(&gK, (size_t)m.slab)) || (rc = S.alloc(&gR, (size_t)m.slab))) return rc;
+    const size_t bytes = sizeof(float) * (size_t)m.slab;
+    HIPTRY(c, hipMemsetAsync(gK, 0, bytes, c->stream));
+    HIPTRY(c, hipMemsetAsync(gR, 0, bytes, c->stream));
+    int64_t gn3[3];
+    shape_of(g.ndim, g.order, g.physics, g.n, GPI_P, gn3);
+
+    // several steps per launch: both wavefields in rings, p of the first one forced inside the
+    // launch, and one imaging launch per group of steps.  One step at a time this loop is bound by
+    // its 7 launches a step (strips, four passes, imaging: about 2.5 us each); 301 x 401 cells, 700
+    // steps with the forward run: 29.9 ms, with the ring 13.1 ms
+    if (c->sample_ev.empty()) {
+        int64_t launches = 0;
+        AdjointRing A1(c), A2(c);
+        rc = A1.take(m, {GPI_P, GPI_VX, GPI_VZ}, false);
+        if (!rc) rc = A2.take(m, {GPI_P, GPI_VX, GPI_VZ}, false);
+        if (rc && rc != GPI_ENOMEM) return rc;
+        Mover B1{c, m, A1.st, A1.ring, src1, XV1, XS1, {}, false, &launches};
+        Mover B2{c, m, A2.st, A2.ring, src2, XV2, XS2, {}, false, &launches};
+        if (!rc && A1.ring.slots == A2.ring.slots &&
+            ((rc = plan_mover(B1, *A1.S, nt, &A1)) || (rc = plan_mover(B2, *A2.S, nt, &A2))))
+            return rc;
+        if (B1.stepped && B2.stepped) {
+            for (int l = 0; l < B1.plan.launches; ++l) {
+                StepParams2D& P = B1.plan.P[l];
+                P.fx = sv.strip[0][2];
+                P.fz = sv.strip[0][0];
+                P.fnt = nt;
+                P.fnp[0] = (int)strip_np(m, 0);
+                P.fnp[1] = (int)strip_np(m, 2);
+            }
+            B1.rewind();
+            B2.rewind();
+            if ((rc = zero_state(c, m, B1.w, c->stream)) || (rc = zero_state(c, m, B2.w, c->stream))) return rc;
+            for (int f : {GPI_P, GPI_VX, GPI_VZ})
+                HIPTRY(c, hipMemcpyAsync(B1.w.field[f], sv.snap[f], bytes, hipMemcpyDeviceToDevice, c->stream));
+            Sampler none(c, nt);
+            HIPTRY(c, hipEventRecord(c->ev[0], c->stream));
+            for (int64_t it = 0; it < nt;) {
+                const int64_t cnt = std::min<int64_t>(A1.steps(), nt - it);
+                const int start = B1.ring.cur;
+                if ((rc = B1.advance(it, cnt)) || (rc = B2.advance(it, cnt))) return rc;
+                image_acoustic_2d_ring(m, B1.ring, B2.ring, start, (int)cnt, gK, gR, dtI, c->stream);
+                ++launches;
+                it += cnt;
+            }
+            if ((rc = finish_timing(c, none, nt, launches))) return rc;
+            if ((rc = download_pitched(c, m, g_invK, gK, gn3)) || (rc = download_pitched(c, m, g_rho, gR, gn3))) return rc;
+            return GPI_OK;
+        }
+    }
+
     // second wavefield: its own wavefields and CPML memory
     struct Held {
         gpi_ctx* c;
@@ -883,23 +972,13 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
             free_allocs(c, st.allocs, st.bytes);
         }
     } h2{c, State{}};
-    int rc = alloc_state(c, m, &h2.st, true);
-    if (rc) return rc;
+    if ((rc = alloc_state(c, m, &h2.st, true))) return rc;
     const State& s2 = h2.st;
-    PassExtras XV1{}, XS1{}, XV2{}, XS2{};
-    Sources src1, src2;
-    if ((rc = plan_sources(c, m, S, shot->nsrc1, shot->src1, shot->wav1, nt, false, XV1, XS1, src1))) return rc;
-    if ((rc = plan_sources(c, m, S, shot->nsrc2, shot->src2, shot->wav2, nt, true, XV2, XS2, src2))) return rc;
-    // previous-step copies (save_tp!) in two alternating sets, and the gradients
+    // previous-step copies (save_tp!) in two alternating sets
     float* tp[2][6];
     for (auto& set : tp)
         for (float*& p : set)
             if ((rc = S.alloc(&p, (size_t)m.slab))) return rc;
-    float *gK, *gR;
-    if ((rc = S.alloc(&gK, (size_t)m.slab)) || (rc = S.alloc(&gR, (size_t)m.slab))) return rc;
-    const size_t bytes = sizeof(float) * (size_t)m.slab;
-    HIPTRY(c, hipMemsetAsync(gK, 0, bytes, c->stream));
-    HIPTRY(c, hipMemsetAsync(gR, 0, bytes, c->stream));
 
     // initial conditions: the first wavefield from the snapshots (boundary_force_snap_tau!,
     // boundary_force_snap_v!, boundary.jl:173-212), the second at rest
@@ -938,9 +1017,7 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
     }
     if ((rc = finish_timing(c, smp, nt, launches))) return rc;
     // the trailing velocity half step of :254-255 changes no output of this mode: omitted
-    int64_t n3[3];
-    shape_of(g.ndim, g.order, g.physics, g.n, GPI_P, n3);
-    if ((rc = download_pitched(c, m, g_invK, gK, n3)) || (rc = download_pitched(c, m, g_rho, gR, n3))) return rc;
+    if ((rc = download_pitched(c, m, g_invK, gK, gn3)) || (rc = download_pitched(c, m, g_rho, gR, gn3))) return rc;
     return GPI_OK;
 }
 

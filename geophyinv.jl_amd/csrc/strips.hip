@@ -48,6 +48,32 @@ __global__ __launch_bounds__(256) void negate_kernel(float* dst, const float* sr
     if (t < n) dst[t] = src[t] * -1.0f;
 }
 
+// The strips of consecutive steps out of a ring of the field: step blockIdx.y's values in slot
+// start + blockIdx.y, its store one strip behind the step's before.
+struct StripRing {
+    StripParams P;
+    const float* ring;
+    int64_t slab;
+    int slots, start;
+};
+
+__global__ __launch_bounds__(256) void strip_ring_kernel(StripRing R)
+{
+    const StripParams& P = R.P;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t n = P.sd0 * P.sd1 * P.sd2;
+    if (t >= n) return;
+    int64_t i = t % P.sd0;
+    const int64_t r = t / P.sd0;
+    int64_t j = r % P.sd1;
+    int64_t k = r / P.sd1;
+    int64_t* ax = P.axis == 0 ? &i : P.axis == 1 ? &j : &k;
+    const int64_t a = *ax;
+    *ax = a < NBOUND ? P.np + a : P.fn_axis - P.np - 2 * NBOUND + a;
+    const int slot = (R.start + (int)blockIdx.y) % R.slots;
+    P.store[t + n * blockIdx.y] = R.ring[R.slab * slot + i + P.p0 * (j + P.p1 * k)] * -1.0f;
+}
+
 // Fields of the imaging condition, in the order p1, vx1, vz1, p2, vx2, vz2 (first and
 // second wavefield).
 struct ImageParams {
@@ -94,6 +120,73 @@ __global__ __launch_bounds__(256) void image2d_kernel(ImageParams P)
     }
 #pragma unroll
     for (int k = 0; k < 6; ++k) P.next[k][o] = P.cur[k][o];
+}
+
+// Bound by the 6 reads per cell and step, nearly all from cache; the two gradients and each
+// wavefield's value that the next step compares with stay in registers, where one launch a step
+// also reads and writes the gradients and copies six arrays.
+// The imaging of image2d_kernel over consecutive steps whose wavefields are rings: slot start + j
+// holds the values before step j, the next slot those after it.
+struct ImageRing {
+    const float* f[6];   // p1, vx1, vz1, p2, vx2, vz2
+    int64_t slab;
+    int slots, start, steps;
+    float* gK;
+    float* gR;
+    int nz, nx, ld, h;
+    float dtI;
+};
+
+__global__ __launch_bounds__(256) void image2d_ring_kernel(ImageRing P)
+{
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    const int j = blockIdx.y * 4 + threadIdx.y;
+    if (i >= P.nz || j >= P.nx) return;
+    const int o = i + P.ld * j;
+    const int h = P.h;
+    const bool rho = i < P.nz - 2 * h && j < P.nx - 2 * h;
+    const int a0 = (i + h) + P.ld * j, a1 = a0 + P.ld;
+    const int b0 = i + P.ld * (j + h), b1 = b0 + 1;
+    const int g = (i + h) + P.ld * (j + h);
+    int slot = P.start;
+    const float* f1 = P.f[0] + P.slab * slot;
+    const float* x1 = P.f[1] + P.slab * slot;
+    const float* z1 = P.f[2] + P.slab * slot;
+    float pp = f1[o], xp0 = 0.0f, xp1 = 0.0f, zp0 = 0.0f, zp1 = 0.0f, gr = 0.0f, gk = P.gK[o];
+    if (rho) {
+        xp0 = x1[a0];
+        xp1 = x1[a1];
+        zp0 = z1[b0];
+        zp1 = z1[b1];
+        gr = P.gR[g];
+    }
+    for (int n = 0; n < P.steps; ++n) {
+        const int next = slot + 1 == P.slots ? 0 : slot + 1;
+        const float p = P.f[0][P.slab * next + o];
+        // compute_gmodKI!: g + p2_prev * (p1_prev - p1) * dtI
+        gk = gk + (P.f[3][P.slab * slot + o] * (pp - p)) * P.dtI;
+        pp = p;
+        if (rho) {
+            const float* vx1 = P.f[1] + P.slab * next;
+            const float* vz1 = P.f[2] + P.slab * next;
+            const float* vx2 = P.f[4] + P.slab * slot;
+            const float* vz2 = P.f[5] + P.slab * slot;
+            const float xc0 = vx1[a0], xc1 = vx1[a1], zc0 = vz1[b0], zc1 = vz1[b1];
+            const float bx0 = (vx2[a0] * (xc0 - xp0)) * P.dtI;
+            const float bx1 = (vx2[a1] * (xc1 - xp1)) * P.dtI;
+            const float bz0 = (vz2[b0] * (zc0 - zp0)) * P.dtI;
+            const float bz1 = (vz2[b1] * (zc1 - zp1)) * P.dtI;
+            // combine_gmodrho!: @inn(g) = @inn(g) - @av_xi(vxbuffer) - @av_zi(vzbuffer)
+            gr = (gr - (bx0 + bx1) * 0.5f) - (bz0 + bz1) * 0.5f;
+            xp0 = xc0;
+            xp1 = xc1;
+            zp0 = zc0;
+            zp1 = zc1;
+        }
+        slot = next;
+    }
+    P.gK[o] = gk;
+    if (rho) P.gR[g] = gr;
 }
 
 // Imaging with the exact forward wavefield, one thread per cell of the pitched slab (z rows
@@ -458,6 +551,53 @@ void image_acoustic_exact(const Model& m, const ImageSets& S, double* g_invK, do
     const int64_t cols = (int64_t)P.py * P.ncol;
     const int64_t nb = (int64_t)((P.ld + 63) / 64) * ((cols + 3) / 4);
     hipLaunchKernelGGL(image_exact_kernel, dim3((unsigned)nb), dim3(64, 4), 0, s, P);
+}
+
+void strip_ring(const Model& m, const Ring& r, int f, const int64_t fn[3], int axis, int64_t np, int start, int steps,
+                float* store, hipStream_t s)
+{
+    StripRing R{};
+    StripParams& P = R.P;
+    P.store = store;
+    int64_t sd[3] = {fn[0], fn[1], fn[2]};
+    sd[axis] = 2 * NBOUND;
+    P.sd0 = sd[0];
+    P.sd1 = sd[1];
+    P.sd2 = sd[2];
+    P.fn_axis = fn[axis];
+    P.np = np;
+    P.p0 = m.pitch0;
+    P.p1 = m.pitch1;
+    P.axis = axis;
+    R.ring = r.base[f];
+    R.slab = r.slab;
+    R.slots = r.slots;
+    R.start = start;
+    const int64_t n = sd[0] * sd[1] * sd[2];
+    hipLaunchKernelGGL(strip_ring_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)steps), dim3(256), 0, s, R);
+}
+
+void image_acoustic_2d_ring(const Model& m, const Ring& r1, const Ring& r2, int start, int steps, float* g_invK,
+                            float* g_rho, float dtI, hipStream_t s)
+{
+    ImageRing P{};
+    const int fs[3] = {GPI_P, GPI_VX, GPI_VZ};
+    for (int q = 0; q < 3; ++q) {
+        P.f[q] = r1.base[fs[q]];
+        P.f[3 + q] = r2.base[fs[q]];
+    }
+    P.slab = r1.slab;
+    P.slots = r1.slots;
+    P.start = start;
+    P.steps = steps;
+    P.gK = g_invK;
+    P.gR = g_rho;
+    P.nz = (int)m.g.n[0];
+    P.nx = (int)m.g.n[2];
+    P.ld = (int)m.pitch0;
+    P.h = m.h;
+    P.dtI = dtI;
+    hipLaunchKernelGGL(image2d_ring_kernel, dim3((P.nz + 63) / 64, (P.nx + 3) / 4), dim3(64, 4), 0, s, P);
 }
 
 void strip_copy(const Model& m, float* field, const int64_t fn[3], int axis, int64_t np, float* store, bool save,
