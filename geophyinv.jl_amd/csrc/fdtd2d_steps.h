@@ -88,6 +88,8 @@ struct StepPlan {
     int cur = 0;             // state that holds the current wavefield
 };
 
+// time steps that one launch takes on this model's grid; 0: such grids are left to the passes
+int launch_steps_2d(const Model& m);
 // Decides whether the shot (its sources and receivers as planned for the passes) can run
 // several steps per launch and prepares it; *ok = false leaves it to the passes.
 int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& src,

@@ -738,6 +738,11 @@ bool pick_tiles(const Model& m, StepTile* all, StepTile* inner)
 }
 
 }  // namespace
+int launch_steps_2d(const Model& m)
+{
+    StepTile all{}, inner{};
+    return m.g.ndim == 2 && pick_tiles(m, &all, &inner) ? all.steps : 0;
+}
 
 int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& src,
                   const gpi_shot* shot, const std::vector<DevPoints>& rec, StepPlan* plan, bool* ok)

@@ -179,9 +179,10 @@ void records_transpose(const float* rec, float* out, int64_t nt, int npts, int* 
 // time-reversal kernels (strips.hip)
 void strip_copy(const Model& m, float* field, const int64_t fn[3], int axis, int64_t np, float* store,
                 bool save, hipStream_t s);
-// boundary_save! of `steps` steps of ring array f, the first one in slot `start`
-void strip_ring(const Model& m, const Ring& r, int f, const int64_t fn[3], int axis, int64_t np, int start, int steps,
-                float* store, hipStream_t s);
+// boundary_save! of `steps` steps of ring array f (2-D, shape fn; np: the z and x strips' width),
+// the first one in slot `start`
+void strip_ring_2d(const Model& m, const Ring& r, int f, const int64_t fn[3], const int64_t np[2], int start, int steps,
+                   float* zstore, float* xstore, hipStream_t s);
 // image_acoustic_2d over `steps` steps of two wavefields in rings (p, vx, vz; the same slots)
 void image_acoustic_2d_ring(const Model& m, const Ring& r1, const Ring& r2, int start, int steps, float* g_invK,
                             float* g_rho, float dtI, hipStream_t s);

@@ -566,13 +566,12 @@ int run_shot(gpi_ctx* c, Model& m, const gpi_shot* shot, Store* save)
         run_steps_2d(m, plan, it, n, c->stream, strips ? &kept : nullptr);
         launches += plan.launches;
         for (int q = 0; strips && q < save->nfield; ++q) {
+            const int64_t np[2] = {strip_np(m, 0), strip_np(m, 2)};
             int64_t fn[3];
             shape_of(g.ndim, g.order, g.physics, g.n, save->field[q], fn);
-            for (int ax = 2; ax >= 0; ax -= 2) {
-                strip_ring(m, kept, save->field[q], fn, ax, strip_np(m, ax), first, n,
-                           save->strip[q][ax] + save->strip_size[q][ax] * it, c->stream);
-                ++launches;
-            }
+            strip_ring_2d(m, kept, save->field[q], fn, np, first, n, save->strip[q][0] + save->strip_size[q][0] * it,
+                          save->strip[q][2] + save->strip_size[q][2] * it, c->stream);
+            ++launches;
         }
         it += n;
         State now = *plan.st[plan.cur];
@@ -734,7 +733,9 @@ struct Mover {
 
 // The adjoint wavefield's arrays over up to IMAGE_STEPS steps, which one imaging launch then
 // reads together; fewer where memory is short, down to the arrays themselves (imaged between
-// the two passes of every step) where `inplace_ok`.
+// the two passes of every step) where `inplace_ok`.  Where a launch takes several steps, as many
+// whole launches as twelve steps hold: with six a launch, 6 + 6 and not 6 + 2 (301 x 401 cells,
+// 700 steps, together with one strip launch for both axes: 13.1 -> 12.0 ms).
 constexpr int IMAGE_STEPS = 8;
 
 struct AdjointRing {
@@ -762,7 +763,9 @@ struct AdjointRing {
     int take(const Model& m, const std::vector<int>& fields, bool inplace_ok)
     {
         int rc = GPI_ENOMEM;
-        for (int n = IMAGE_STEPS; n >= (inplace_ok ? 0 : 1) && rc == GPI_ENOMEM; n /= 2) {
+        const int launch = launch_steps_2d(m);
+        const int most = launch > 1 ? 12 / launch * launch : IMAGE_STEPS;
+        for (int n = most; n >= (inplace_ok ? 0 : 1) && rc == GPI_ENOMEM; n /= 2) {
             drop();
             S = new Scratch(c);
             rc = alloc_ring(c, *S, m, ring, fields, n + 1);
@@ -920,7 +923,7 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
     // several steps per launch: both wavefields in rings, p of the first one forced inside the
     // launch, and one imaging launch per group of steps.  One step at a time this loop is bound by
     // its 7 launches a step (strips, four passes, imaging: about 2.5 us each); 301 x 401 cells, 700
-    // steps with the forward run: 29.9 ms, with the ring 13.1 ms
+    // steps with the forward run: 29.9 ms, with the rings 12.0 ms
     if (c->sample_ev.empty()) {
         int64_t launches = 0;
         AdjointRing A1(c), A2(c);

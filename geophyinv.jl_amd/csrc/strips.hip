@@ -48,10 +48,11 @@ __global__ __launch_bounds__(256) void negate_kernel(float* dst, const float* sr
     if (t < n) dst[t] = src[t] * -1.0f;
 }
 
-// The strips of consecutive steps out of a ring of the field: step blockIdx.y's values in slot
-// start + blockIdx.y, its store one strip behind the step's before.
+// Both axes' strips of consecutive steps out of a ring of a 2-D field: step blockIdx.y's values
+// in slot start + blockIdx.y, its store one strip behind the step's before.  Bound by the launch
+// (6 planes a side of each axis): one for 2 axes x 6 steps instead of one each.
 struct StripRing {
-    StripParams P;
+    StripParams P[2];   // z, x
     const float* ring;
     int64_t slab;
     int slots, start;
@@ -59,19 +60,18 @@ struct StripRing {
 
 __global__ __launch_bounds__(256) void strip_ring_kernel(StripRing R)
 {
-    const StripParams& P = R.P;
+    const bool xs = blockIdx.z != 0;
+    const StripParams& P = R.P[xs ? 1 : 0];
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n = P.sd0 * P.sd1 * P.sd2;
+    const int64_t n = P.sd0 * P.sd2;
     if (t >= n) return;
     int64_t i = t % P.sd0;
-    const int64_t r = t / P.sd0;
-    int64_t j = r % P.sd1;
-    int64_t k = r / P.sd1;
-    int64_t* ax = P.axis == 0 ? &i : P.axis == 1 ? &j : &k;
-    const int64_t a = *ax;
-    *ax = a < NBOUND ? P.np + a : P.fn_axis - P.np - 2 * NBOUND + a;
+    int64_t k = t / P.sd0;
+    const int64_t a = xs ? k : i;
+    const int64_t c = a < NBOUND ? P.np + a : P.fn_axis - P.np - 2 * NBOUND + a;
+    (xs ? k : i) = c;
     const int slot = (R.start + (int)blockIdx.y) % R.slots;
-    P.store[t + n * blockIdx.y] = R.ring[R.slab * slot + i + P.p0 * (j + P.p1 * k)] * -1.0f;
+    P.store[t + n * blockIdx.y] = R.ring[R.slab * slot + i + P.p0 * k] * -1.0f;
 }
 
 // Fields of the imaging condition, in the order p1, vx1, vz1, p2, vx2, vz2 (first and
@@ -553,28 +553,26 @@ void image_acoustic_exact(const Model& m, const ImageSets& S, double* g_invK, do
     hipLaunchKernelGGL(image_exact_kernel, dim3((unsigned)nb), dim3(64, 4), 0, s, P);
 }
 
-void strip_ring(const Model& m, const Ring& r, int f, const int64_t fn[3], int axis, int64_t np, int start, int steps,
-                float* store, hipStream_t s)
+void strip_ring_2d(const Model& m, const Ring& r, int f, const int64_t fn[3], const int64_t np[2], int start, int steps,
+                   float* zstore, float* xstore, hipStream_t s)
 {
     StripRing R{};
-    StripParams& P = R.P;
-    P.store = store;
-    int64_t sd[3] = {fn[0], fn[1], fn[2]};
-    sd[axis] = 2 * NBOUND;
-    P.sd0 = sd[0];
-    P.sd1 = sd[1];
-    P.sd2 = sd[2];
-    P.fn_axis = fn[axis];
-    P.np = np;
-    P.p0 = m.pitch0;
-    P.p1 = m.pitch1;
-    P.axis = axis;
+    int64_t n = 0;
+    for (int q = 0; q < 2; ++q) {
+        StripParams& P = R.P[q];
+        P.store = q ? xstore : zstore;
+        P.sd0 = q ? fn[0] : 2 * NBOUND;
+        P.sd2 = q ? 2 * NBOUND : fn[2];
+        P.fn_axis = fn[2 * q];
+        P.np = np[q];
+        P.p0 = m.pitch0;
+        n = std::max(n, P.sd0 * P.sd2);
+    }
     R.ring = r.base[f];
     R.slab = r.slab;
     R.slots = r.slots;
     R.start = start;
-    const int64_t n = sd[0] * sd[1] * sd[2];
-    hipLaunchKernelGGL(strip_ring_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)steps), dim3(256), 0, s, R);
+    hipLaunchKernelGGL(strip_ring_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)steps, 2), dim3(256), 0, s, R);
 }
 
 void image_acoustic_2d_ring(const Model& m, const Ring& r1, const Ring& r2, int start, int steps, float* g_invK,
