@@ -178,6 +178,80 @@ __device__ __forceinline__ void str_ac_point(const StrParams2D& P, const PassExt
     into<RING>(P.s0, P.out)[o] = p;
 }
 
+// RX columns j0 .. j0 + RX - 1 of row i, all of them inside the ranges of both velocities: along
+// x they share all but one of each other's samples.
+template <int O, int RX, bool RING>
+__device__ __forceinline__ void vel_ac_columns(const VelParams2D& P, const PassExtras& X, int64_t it, int ninj, int i,
+                                               int j0)
+{
+    constexpr int H = O - 1;
+    const int ld = P.ld;
+    float px[O + RX - 1], pz[RX][O], vxo[RX], vzo[RX], rx[RX + 1], rz0[RX], rz1[RX];
+    load_x<O + RX - 1>(px, P.s0, (i + H) + ld * j0, ld);
+    load_x<RX + 1>(rx, P.rho, (i + H) + ld * j0, ld);
+#pragma unroll
+    for (int r = 0; r < RX; ++r) {
+        const int c = i + ld * (j0 + r + H);
+        load_z<O>(pz[r], P.s0, c);
+        vxo[r] = P.vx[c + H];
+        vzo[r] = P.vz[c + H];
+        rz0[r] = P.rho[c];
+        rz1[r] = P.rho[c + 1];
+    }
+#pragma unroll
+    for (int r = 0; r < RX; ++r) {
+        const int j = j0 + r;
+        const int o = (i + H) + ld * (j + H);
+        const int bk = (i >> 6) + P.gx * j;
+        const float cxo = dt_over_av2(P.dt, rx[r], rx[r + 1]);    // dtinvavxirho
+        const float czo = dt_over_av2(P.dt, rz0[r], rz1[r]);      // dtinvavzirho
+        float d = stencil<O>(px + r) * P.dxI;
+        d = cpml_x(d, P.qx0, i, j, P.npml, P.pml_mask);
+        float nv = vxo[r] + cxo * d;
+        if ((P.rigid_mask & GPI_FACE(2, 0)) && j == 0) into<RING>(P.vx, P.out)[(i + H)] = -nv;
+        if (ninj) nv = inject_velocity(X, it, INJ_VX, bk, o, nv, P.rho, P.dt);
+        into<RING>(P.vx, P.out)[o] = nv;
+        d = stencil<O>(pz[r]) * P.dzI;
+        d = cpml_z(d, P.qz0, i, j, P.npml, P.pml_mask);
+        nv = vzo[r] + czo * d;
+        if ((P.rigid_mask & GPI_FACE(0, 0)) && i == 0) into<RING>(P.vz, P.out)[ld * (j + H)] = -nv;
+        if (ninj) nv = inject_velocity(X, it, INJ_VZ, bk, o, nv, P.rho, P.dt);
+        into<RING>(P.vz, P.out)[o] = nv;
+    }
+}
+
+template <int O, int RX, bool RING>
+__device__ __forceinline__ void str_ac_columns(const StrParams2D& P, const PassExtras& X, int64_t it, int ninj, int i,
+                                               int j0)
+{
+    const int ld = P.ld;
+    const int o0 = i + ld * j0;
+    float vxs[O + RX - 1], vzs[RX][O], c[RX], po[RX];
+    load_x<O + RX - 1>(vxs, P.vx, o0, ld);
+#pragma unroll
+    for (int r = 0; r < RX; ++r) {
+        load_z<O>(vzs[r], P.vz, o0 + r * ld);
+        c[r] = P.c0[o0 + r * ld];
+        po[r] = P.s0[o0 + r * ld];
+    }
+#pragma unroll
+    for (int r = 0; r < RX; ++r) {
+        const int j = j0 + r, o = o0 + r * ld;
+        float dvx = stencil<O>(vxs + r) * P.dxI;         // D_xa(vx)
+        dvx = cpml_x(dvx, P.qx0, i, j, P.npml, P.pml_mask);
+        float dvz = stencil<O>(vzs[r]) * P.dzI;          // D_za(vz)
+        dvz = cpml_z(dvz, P.qz0, i, j, P.npml, P.pml_mask);
+        float p = po[r] + (dvx + dvz) * c[r];
+        const int bk = (i >> 6) + P.gx * j;
+        for (int q = 0; q < ninj; ++q) {
+            float acc;
+            int t;
+            if (X.inj[q].kind == INJ_P && injection_sum(X.inj[q], bk, o, it, acc, t)) p = p + (acc * c[r]);
+        }
+        into<RING>(P.s0, P.out)[o] = p;
+    }
+}
+
 // Elastic updates from their operands (the point functions below load them).
 template <int O>
 __device__ __forceinline__ float vel_el_vx(const VelParams2D& P, int i, int j, const float (&a1)[O],
@@ -343,6 +417,12 @@ __device__ __forceinline__ void vel_tile(const VelParams2D& P, const PassExtras&
 {
     const int i = (b % P.gx) * 64 + (int)threadIdx.x;
     const int j0 = (b / P.gx) * (TY * RX) + (int)threadIdx.y * RX;
+    if constexpr (PHYS == 0 && RX > 1) {
+        if (i < P.nz - 2 * (O - 1) && j0 + RX <= P.nx - 2 * (O - 1)) {
+            vel_ac_columns<O, RX, RING>(P, X, it, ninj, i, j0);
+            return;
+        }
+    }
 #pragma unroll
     for (int r = 0; r < RX; ++r) {
         if (PHYS == 0) vel_ac_point<O, RING>(P, X, it, ninj, i, j0 + r);
@@ -355,6 +435,12 @@ __device__ __forceinline__ void str_tile(const StrParams2D& P, const PassExtras&
 {
     const int i = (b % P.gx) * 64 + (int)threadIdx.x;
     const int j0 = (b / P.gx) * (TY * RX) + (int)threadIdx.y * RX;
+    if constexpr (PHYS == 0 && RX > 1) {
+        if (i < P.nz && j0 + RX <= P.nx) {
+            str_ac_columns<O, RX, RING>(P, X, it, ninj, i, j0);
+            return;
+        }
+    }
 #pragma unroll
     for (int r = 0; r < RX; ++r) {
         if (PHYS == 0) str_ac_point<O, RING>(P, X, it, ninj, i, j0 + r);
@@ -363,20 +449,25 @@ __device__ __forceinline__ void str_tile(const StrParams2D& P, const PassExtras&
 }
 
 // ---------------------------------------------------------------------------------------
-// One shot per launch (the drop-in path): 64 x 4 workgroups, one column per thread.
+// One shot per launch (the drop-in path).
 // ---------------------------------------------------------------------------------------
 
-// Workgroup shape of the single-shot kernels: index into TILE_SHAPES, from GPI_TILE2D
-// (default 0: 64 x 4 threads, one column each).
-int plain_shape()
+// Workgroup shape of the single-shot kernels: index into TILE_SHAPES, from GPI_TILE2D if set,
+// else 64 x 4 threads of one column each.  Acoustic passes of orders 4 to 8 on large grids give
+// each thread two columns, which share their samples along x (vel_ac_columns, str_ac_columns):
+// there the loads of a stencil's 2 x O neighbours bound the pass.  On smaller grids, whose arrays
+// stay in the XCDs' L2, half the waves hide less latency.  us per step, one / two columns:
+// order 8, 942 x 1243 cells 16.7 / 17.7, 1142 x 1243 18.7 / 18.8, 1292 x 1243 20.8 / 20.1,
+// 1842 x 1243 26.9 / 25.2, 2642 x 1443 39.1 / 35.3; order 6 the same within 3 %; order 4,
+// 942 x 1243 15.4 / 16.3, 1842 x 1243 25.3 / 23.9.
+int plain_shape(int order, int physics, int64_t cells)
 {
-    static int t = -1;
-    if (t < 0) {
+    static const int set = [] {
         const char* e = getenv("GPI_TILE2D");
-        t = e ? atoi(e) : 0;
-        if (t < 0 || t > 3) t = 0;
-    }
-    return t;
+        const int t = e ? atoi(e) : -1;
+        return e && (t < 0 || t > 3) ? 0 : t;
+    }();
+    return set >= 0 ? set : physics == 0 && order >= 4 && cells >= 1500000 ? 2 : 0;
 }
 
 template <int O, int PHYS, int TY, int RX, bool RING>
@@ -425,7 +516,7 @@ void launch_plain(bool velocity, hipStream_t s, VelParams2D V, StrParams2D S, co
 template <int O, int PHYS>
 void launch_plain_o(bool velocity, hipStream_t s, const VelParams2D& V, const StrParams2D& S, const PassExtras& X)
 {
-    switch (plain_shape()) {
+    switch (plain_shape(O, PHYS, velocity ? (int64_t)V.nz * V.nx : (int64_t)S.nz * S.nx)) {
     case 1: launch_plain<O, PHYS, 8, 1>(velocity, s, V, S, X); break;
     case 2: launch_plain<O, PHYS, 2, 2>(velocity, s, V, S, X); break;
     case 3: launch_plain<O, PHYS, 4, 2>(velocity, s, V, S, X); break;
