@@ -475,7 +475,9 @@ int gpi_conv_lsmr(gpi_ctx* ctx, int64_t nt, int64_t ntr, const double* g, const 
 int gpi_last_timing(const gpi_ctx* ctx, gpi_timing* out);
 
 /* Bracket the velocity and stress passes of up to `nsamples` evenly spaced steps of each
- * following gpi_forward with HIP events (0 turns sampling off).  No reference counterpart:
+ * following gpi_forward with HIP events (0 turns sampling off).  A sampled 2-D shot runs one
+ * pass per launch; otherwise 2-D shots take several steps per launch where they can, with the
+ * same results, and there is no pass to time.  No reference counterpart:
  * it replaces the TimerOutputs sections of src/fdtd/propagate.jl:176-232 with device
  * time. */
 int gpi_set_pass_sampling(gpi_ctx* ctx, int32_t nsamples);
