@@ -68,12 +68,19 @@ struct BatchShot2D {
     int64_t nt;
 };
 
+// Workgroups of a batched launch as shot << 16 | workgroup of the shot, in the order of dispatch
+// over the XCDs; BATCH_NONE past the last.  Launches of at most BATCH_MAP workgroups read it.
+constexpr uint32_t BATCH_NONE = ~0u;
+constexpr int BATCH_MAP = 1 << 15;
+void batch_map(const int* first, int n, int launch, uint32_t* map);
+
 // One pass of every shot of a device table: n = *nshots shots, first[s] = first workgroup
 // of shot s, first[n] = the workgroups they need; the launch has nblocks >= first[n]
-// workgroups.  All shots share physics, order and tile shape.
+// workgroups, found by `map` or, if it is null, by a search over `first`.  All shots share
+// physics, order and tile shape.
 void batch_pass_2d(int physics, int order, const TileShape& t, bool velocity, const BatchShot2D* D,
-                   const int* first, const int* nshots, int nblocks, const int64_t* step0, int koff,
-                   hipStream_t s);
+                   const int* first, const int* nshots, int nblocks, const uint32_t* map, const int64_t* step0,
+                   int koff, hipStream_t s);
 // *step0 = step, stream-ordered (a one-thread kernel: no memset node in a captured chunk).
 void batch_set_step(int64_t* step0, int64_t step, hipStream_t s);
 

@@ -177,6 +177,8 @@ struct gpi_server {
     PinnedPool pool;
     BatchShot2D* dtab = nullptr;
     int* dfirst = nullptr;
+    uint32_t* dmap = nullptr;                  // workgroup maps of the velocity and stress launches
+    uint32_t* hmap[2] = {nullptr, nullptr};
     char* htab[2] = {nullptr, nullptr};
     hipEvent_t tab_ev[2] = {nullptr, nullptr};
     int tab_cur = 0;
@@ -280,8 +282,10 @@ void gpi_server::launch_chunk(const TileShape& t, int nbv, int nbs, int64_t K, h
 {
     const int* nsh = dfirst + 2 * (o.max_shots + 1);
     for (int64_t k = 0; k < K; ++k) {
-        batch_pass_2d(o.physics, o.order, t, true, dtab, dfirst, nsh, nbv, dstep, (int)k, st);
-        batch_pass_2d(o.physics, o.order, t, false, dtab, dfirst + o.max_shots + 1, nsh, nbs, dstep, (int)k, st);
+        batch_pass_2d(o.physics, o.order, t, true, dtab, dfirst, nsh, nbv, nbv <= BATCH_MAP ? dmap : nullptr, dstep,
+                      (int)k, st);
+        batch_pass_2d(o.physics, o.order, t, false, dtab, dfirst + o.max_shots + 1, nsh, nbs,
+                      nbs <= BATCH_MAP ? dmap + BATCH_MAP : nullptr, dstep, (int)k, st);
     }
 }
 
@@ -514,6 +518,15 @@ int gpi_server::upload_table(const TileShape& t, int* nbv, int* nbs)
     HIPTRY(cc, hipMemcpyAsync(dtab, T, sizeof(BatchShot2D) * n, hipMemcpyHostToDevice, cc->stream));
     HIPTRY(cc, hipMemcpyAsync(dfirst, fv, sizeof(int) * (2 * (o.max_shots + 1) + 1), hipMemcpyHostToDevice,
                               cc->stream));
+    for (int q = 0; q < 2; ++q) {   // whole buckets: captured launches cover them
+        const int* f = q ? fs : fv;
+        const int launch = std::min(launch_bucket(f[n]), BATCH_MAP);
+        if (f[n] > BATCH_MAP) continue;
+        uint32_t* map = hmap[tab_cur] + q * BATCH_MAP;
+        batch_map(f, n, launch, map);
+        HIPTRY(cc, hipMemcpyAsync(dmap + q * BATCH_MAP, map, sizeof(uint32_t) * (size_t)launch, hipMemcpyHostToDevice,
+                                  cc->stream));
+    }
     HIPTRY(cc, hipEventRecord(tab_ev[tab_cur], cc->stream));
     tab_cur ^= 1;
     *nbv = nv;
@@ -795,11 +808,13 @@ int gpi_server_create(int device, const gpi_server_opts* opts, gpi_server** out)
     const size_t tb = sizeof(BatchShot2D) * v->o.max_shots + sizeof(int) * (2 * (v->o.max_shots + 1) + 1);
     bool ok = hipMalloc((void**)&v->dtab, sizeof(BatchShot2D) * v->o.max_shots) == hipSuccess &&
               hipMalloc((void**)&v->dfirst, sizeof(int) * (2 * (v->o.max_shots + 1) + 1)) == hipSuccess &&
+              hipMalloc((void**)&v->dmap, sizeof(uint32_t) * 2 * BATCH_MAP) == hipSuccess &&
               hipMalloc((void**)&v->dstep, sizeof(int64_t)) == hipSuccess &&
               hipStreamCreateWithFlags(&v->cap, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreateWithFlags(&v->adm_ev, hipEventDisableTiming) == hipSuccess;
     for (int k = 0; k < 2 && ok; ++k) {
         ok = hipHostMalloc((void**)&v->htab[k], tb, hipHostMallocDefault) == hipSuccess &&
+             hipHostMalloc((void**)&v->hmap[k], sizeof(uint32_t) * 2 * BATCH_MAP, hipHostMallocDefault) == hipSuccess &&
              hipEventCreateWithFlags(&v->tab_ev[k], hipEventDisableTiming) == hipSuccess &&
              hipEventCreate(&v->ck_ev[k][0]) == hipSuccess && hipEventCreate(&v->ck_ev[k][1]) == hipSuccess;
         if (ok) ok = hipEventRecord(v->tab_ev[k], v->cc->stream) == hipSuccess;
@@ -842,9 +857,11 @@ void gpi_server_destroy(gpi_server* v)
     if (v->cap) (void)hipStreamDestroy(v->cap);
     if (v->dtab) (void)hipFree(v->dtab);
     if (v->dfirst) (void)hipFree(v->dfirst);
+    if (v->dmap) (void)hipFree(v->dmap);
     if (v->dstep) (void)hipFree(v->dstep);
     for (int k = 0; k < 2; ++k) {
         if (v->htab[k]) (void)hipHostFree(v->htab[k]);
+        if (v->hmap[k]) (void)hipHostFree(v->hmap[k]);
         if (v->tab_ev[k]) (void)hipEventDestroy(v->tab_ev[k]);
         for (int e = 0; e < 2; ++e)
             if (v->ck_ev[k][e]) (void)hipEventDestroy(v->ck_ev[k][e]);
