@@ -1,5 +1,7 @@
 // Several time steps of one 2-D shot per launch (fdtd2d_steps.hip).
 #pragma once
+#include <memory>
+
 #include "gpi_util.h"
 
 namespace gpi {
@@ -84,6 +86,7 @@ struct StepPlan {
     bool inner[2] = {};
     StepParams2D P[2] = {};
     State* st[2] = {};
+    std::shared_ptr<State> alt;   // the second of them (its memory in the call's scratch)
     int ders[8] = {};        // derivative fields of psi_in
     int cur = 0;             // state that holds the current wavefield
 };
@@ -91,10 +94,11 @@ struct StepPlan {
 // time steps that one launch takes on this model's grid; 0: such grids are left to the passes
 int launch_steps_2d(const Model& m);
 // Decides whether the shot (its sources and receivers as planned for the passes) can run
-// several steps per launch and prepares it; *ok = false leaves it to the passes.
+// several steps per launch and prepares it in memory of S; *ok = false leaves it to the passes.
+// Without `second` the caller names both states itself.
 int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& src,
                   const gpi_shot* shot, const std::vector<DevPoints>& rec, StepPlan* plan,
-                  bool* ok);
+                  bool* ok, bool second = true);
 // `steps` <= plan.steps time steps from it0; the arrays of `ring` (if given) take the slots
 // after its current one instead of the two states
 void run_steps_2d(const Model& m, StepPlan& plan, int64_t it0, int steps, hipStream_t s, Ring* ring = nullptr);

@@ -745,7 +745,7 @@ int launch_steps_2d(const Model& m)
 }
 
 int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& src,
-                  const gpi_shot* shot, const std::vector<DevPoints>& rec, StepPlan* plan, bool* ok)
+                  const gpi_shot* shot, const std::vector<DevPoints>& rec, StepPlan* plan, bool* ok, bool second)
 {
     *ok = false;
     const gpi_grid& g = m.g;
@@ -924,34 +924,29 @@ int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& s
     for (size_t k = 0; k < rl.size(); ++k)
         std::memcpy(&tab[sr + sizeof(TileReceiver) * k], &rl[k].second, sizeof(TileReceiver));
 
-    // ---- the second state and the coefficients: without room for them the passes run
-    if (!m.st1) {
-        State* st = new State();
-        float* co[5] = {};
-        int rc = alloc_state(c, m, st);
-        for (int k = 0; !rc && k < (ac ? 2 : 5); ++k) {
-            void* p = nullptr;
-            rc = dev_alloc(c, &st->allocs, &st->bytes, &p, sizeof(float) * (size_t)m.slab);
-            co[k] = (float*)p;
-        }
-        if (rc) {
-            free_state(c, st);
-            (void)hipGetLastError();
-            c->err.clear();
-            return GPI_OK;
-        }
-        m.st1 = st;
-        std::copy(co, co + 5, m.step_coef);
-    }
-    int rc;
+    // ---- the second state, the coefficients and the tables, for this call alone: without room for
+    // them the passes run
+    Scratch R(c);
+    auto alt = std::make_shared<State>();
+    float* co[5] = {};
     char* dtab = nullptr;
     float* amp = nullptr;
-    if ((rc = S.put(&dtab, tab))) return rc;
+    int rc = second ? alloc_state(c, m, alt.get(), true) : GPI_OK;
+    R.p.swap(alt->allocs);
+    std::swap(R.bytes, alt->bytes);
+    for (int k = 0; !rc && k < (ac ? 2 : 5); ++k) rc = R.alloc(&co[k], (size_t)m.slab);
+    if (!rc && namp) rc = R.alloc(&amp, (size_t)namp * (size_t)nt);
+    if (!rc) rc = R.put(&dtab, tab);
+    if (rc == GPI_ENOMEM) {
+        (void)hipGetLastError();
+        c->err.clear();
+        return GPI_OK;
+    }
+    if (rc) return rc;
     P.box = (const TileBox*)dtab;
     P.src = (const TileSource*)(dtab + sb);
     P.rec = (const TileReceiver*)(dtab + sr);
     P.ntile = ntile;
-    float* const* co = m.step_coef;
     const dim3 grd((nz + H + 63) / 64, (nx + H + 3) / 4), blk(64, 4);
     if (ac)
         hipLaunchKernelGGL(step_coef_kernel<0>, grd, blk, 0, c->stream, m.coef[GPI_C_RHO], (const float*)nullptr,
@@ -966,7 +961,6 @@ int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& s
     P.coef[3] = co[3];
     P.coef[4] = co[4];
     if (namp) {
-        if ((rc = S.alloc(&amp, (size_t)namp * (size_t)nt))) return rc;
         int base = 0;
         for (const DevPoints& D : src.pts) {
             if (D.ntarget == 0) continue;
@@ -1010,7 +1004,12 @@ int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& s
     plan->tile[plan->launches] = t[0];
     plan->inner[plan->launches++] = false;
     plan->st[0] = m.st0;
-    plan->st[1] = m.st1;
+    plan->alt = alt;
+    plan->st[1] = second ? alt.get() : nullptr;
+    S.p.insert(S.p.end(), R.p.begin(), R.p.end());
+    S.bytes += R.bytes;
+    R.p.clear();
+    R.bytes = 0;
     plan->cur = 0;
     std::copy(ders, ders + 8, plan->ders);
     *ok = true;

@@ -67,8 +67,6 @@ struct Model {
     Pml pml[GPI_NFIELDS];              // strides and coefficient vectors; psi lives in a State
     float* pmlvec = nullptr;           // all a, b, kI vectors
     State* st0 = nullptr;              // the state of gpi_forward / gpi_forward_save
-    State* st1 = nullptr;              // 2-D: the state that several-step launches alternate with (made when first used)
-    float* step_coef[5] = {};          // their coefficients (owned by st1)
 };
 
 // Wavefields that keep their last `slots` values: array f is base[f] with one slab per slot,

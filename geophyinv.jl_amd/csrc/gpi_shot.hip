@@ -783,7 +783,7 @@ int plan_mover(Mover& M, Scratch& S, int64_t nt, AdjointRing* adj)
 {
     gpi_ctx* c = M.c;
     if (M.m.g.ndim != 2 || (adj && adj->inplace())) return GPI_OK;
-    int rc = plan_steps_2d(c, const_cast<Model&>(M.m), S, nt, M.src, nullptr, {}, &M.plan, &M.stepped);
+    int rc = plan_steps_2d(c, const_cast<Model&>(M.m), S, nt, M.src, nullptr, {}, &M.plan, &M.stepped, !adj);
     if (rc || !M.stepped) return rc;
     if (adj) {
         if ((rc = alloc_state(c, M.m, &adj->alt, true, &adj->ring))) {

@@ -218,7 +218,6 @@ void free_state(gpi_ctx* c, State* st)
 void free_model(gpi_ctx* c, Model* m)
 {
     free_state(c, m->st0);
-    free_state(c, m->st1);
     free_allocs(c, m->allocs, m->bytes);
     delete m;
 }
