@@ -118,7 +118,14 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
     if (RZ == 64) g = __builtin_amdgcn_readfirstlane(g);
     const int lc0 = g * K;
     const int czl = B.z0, czh = B.z1, cxl = B.x0, cxh = B.x1;
-    const int r0 = czl - P.lead, c0 = cxl - P.lead;
+    // Cores are dealt evenly, so a small one's tile reaches past its own halo.  Inner tiles load
+    // every cell without a test: their last ones start earlier instead of ending outside the grid
+    // (the cells between are further halo, and inner tiles have no table of cells).
+    int r0 = czl - P.lead, c0 = cxl - P.lead;
+    if constexpr (!SR) {
+        r0 = min(r0, P.nz + H - RZ);
+        c0 = min(c0, P.nx + H - WX);
+    }
     const int r = r0 + lr, cc = c0 + lc0;
     const int ld = P.ld;
     float* const L = Q.f + T::PAD + lr + RZ * lc0;   // this thread's first cell of array 0
@@ -297,8 +304,8 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
         }
         const float* amp = Q.amp + (s & 1) * MAX_TILE_SOURCES;
         // columns whose values are still needed: the rest of the halo is stale already
-        const int need0 = P.lead - (P.steps - 1 - s) * H;
-        const int need1 = P.lead + (cxh - cxl) + (P.steps - s) * H;
+        const int need0 = (cxl - c0) - (P.steps - 1 - s) * H;
+        const int need1 = (cxh - c0) + (P.steps - s) * H;
         gather(false, it);
         if (lc0 + K > need0 && lc0 < need1) {
             if (PP && edge) {   // the free surface's row is written by the row below
