@@ -919,6 +919,8 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
     HIPTRY(c, hipMemsetAsync(gR, 0, bytes, c->stream));
     int64_t gn3[3];
     shape_of(g.ndim, g.order, g.physics, g.n, GPI_P, gn3);
+    float* pack;   // of the downloads: before the rings, which take what is left
+    if ((rc = S.alloc(&pack, (size_t)(gn3[0] * gn3[1] * gn3[2])))) return rc;
 
     // several steps per launch: both wavefields in rings, p of the first one forced inside the
     // launch, and one imaging launch per group of steps.  One step at a time this loop is bound by
@@ -960,7 +962,8 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
                 it += cnt;
             }
             if ((rc = finish_timing(c, none, nt, launches))) return rc;
-            if ((rc = download_pitched(c, m, g_invK, gK, gn3)) || (rc = download_pitched(c, m, g_rho, gR, gn3))) return rc;
+            if ((rc = download_pitched(c, m, g_invK, gK, gn3, pack)) || (rc = download_pitched(c, m, g_rho, gR, gn3, pack)))
+                return rc;
             return GPI_OK;
         }
     }
@@ -1020,7 +1023,7 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
     }
     if ((rc = finish_timing(c, smp, nt, launches))) return rc;
     // the trailing velocity half step of :254-255 changes no output of this mode: omitted
-    if ((rc = download_pitched(c, m, g_invK, gK, gn3)) || (rc = download_pitched(c, m, g_rho, gR, gn3))) return rc;
+    if ((rc = download_pitched(c, m, g_invK, gK, gn3, pack)) || (rc = download_pitched(c, m, g_rho, gR, gn3, pack))) return rc;
     return GPI_OK;
 }
 
@@ -1081,17 +1084,18 @@ int gpi_adjoint_checkpoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi
     const size_t bytes = sizeof(float) * slab;
     int64_t launches = 0;
     // the segment's forward wavefield: p_{n0-1} .. p_{n1-1} in slots 0 .. L and, for rho, v_{n0-1}
-    // .. v_{n1} in slots 0 .. L + 1, the last one from the segment after it
+    // .. v_{n1} in slots 0 .. L + 1, the last one (which the steps do not reach) from the segment
+    // after it
     Mover F{c, m, *m.st0, {}, R.src, R.xv, R.xs, {}, false, &launches};
     if ((rc = alloc_ring(c, S, m, F.ring, {GPI_P}, (int)(L + 1)))) return rc;
     if (rho && (rc = alloc_ring(c, S, m, F.ring, vf, (int)(L + 2)))) return rc;
-    float* vnext[GPI_NFIELDS] = {};
-    if (rho)
-        for (int f : vf)
-            if ((rc = S.alloc(&vnext[f], slab))) return rc;
     double *gK = nullptr, *gR = nullptr;
     if ((rc = S.alloc(&gK, slab))) return rc;
     if (rho && (rc = S.alloc(&gR, slab))) return rc;
+    int64_t n3[3];
+    shape_of(g.ndim, g.order, g.physics, g.n, GPI_P, n3);
+    double* pack;   // of the downloads: before the adjoint ring, which takes what is left
+    if ((rc = S.alloc(&pack, (size_t)(n3[0] * n3[1] * n3[2])))) return rc;
     // the adjoint wavefield: p before and (for rho) v around up to IMAGE_STEPS steps
     AdjointRing A(c);
     std::vector<int> kept{GPI_P};
@@ -1106,7 +1110,9 @@ int gpi_adjoint_checkpoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi
     B.rewind();
     if ((rc = zero_state(c, m, B.w, c->stream))) return rc;
     if (rho)   // v_nt: the trailing half step of the stored run
-        for (int f : vf) HIPTRY(c, hipMemcpyAsync(vnext[f], sv.snap[f], bytes, hipMemcpyDeviceToDevice, c->stream));
+        for (int f : vf)
+            HIPTRY(c, hipMemcpyAsync(F.ring.base[f] + (size_t)(nt - (K - 1) * C + 1) * slab, sv.snap[f], bytes,
+                                     hipMemcpyDeviceToDevice, c->stream));
 
     Sampler smp(c, nt);
     int64_t it = 0;
@@ -1118,10 +1124,6 @@ int gpi_adjoint_checkpoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi
         if (k == 0) rc = zero_state(c, m, F.w, c->stream);
         else rc = copy_state(c, m, F.w, sv.ckpt[k - 1], false, c->stream);
         if (rc || (rc = F.advance(n0, n1 - n0))) return rc;
-        if (rho)
-            for (int f : vf)
-                HIPTRY(c, hipMemcpyAsync(F.ring.base[f] + (size_t)(n1 - n0 + 1) * slab, vnext[f], bytes,
-                                         hipMemcpyDeviceToDevice, c->stream));
         // the adjoint steps of this segment, forward step n = nt - 1 - it, and their imaging
         for (int64_t n = n1 - 1; n >= n0;) {
             const int64_t cnt = std::min<int64_t>(A.steps(), n - n0 + 1);
@@ -1146,15 +1148,14 @@ int gpi_adjoint_checkpoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi
             it += cnt;
             n -= cnt;
         }
-        if (rho)
+        if (rho && k)   // v_{n0} for the segment before it, which has C = L steps
             for (int f : vf)
-                HIPTRY(c, hipMemcpyAsync(vnext[f], F.ring.base[f] + slab, bytes, hipMemcpyDeviceToDevice, c->stream));
+                HIPTRY(c, hipMemcpyAsync(F.ring.base[f] + (size_t)(L + 1) * slab, F.ring.base[f] + slab, bytes,
+                                         hipMemcpyDeviceToDevice, c->stream));
     }
     if ((rc = finish_timing(c, smp, nt, launches))) return rc;
-    int64_t n3[3];
-    shape_of(g.ndim, g.order, g.physics, g.n, GPI_P, n3);
-    if ((rc = download_pitched(c, m, g_invK, gK, n3))) return rc;
-    if (rho && (rc = download_pitched(c, m, g_rho, gR, n3))) return rc;
+    if ((rc = download_pitched(c, m, g_invK, gK, n3, pack))) return rc;
+    if (rho && (rc = download_pitched(c, m, g_rho, gR, n3, pack))) return rc;
     return GPI_OK;
 }
 
@@ -1250,15 +1251,6 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
     E.P = acc[1];
     for (int q = 0; q < E.ns; ++q) E.S[q] = acc[2 + q];
     for (int q = 0; q < E.nv; ++q) E.R[q] = acc[2 + E.ns + q];
-    // the adjoint wavefield: its arrays around up to IMAGE_STEPS steps
-    AdjointRing A(c);
-    if ((rc = A.take(m, all, true))) return rc;
-    Mover B{c, m, A.st, A.ring, src2, XV2, XS2, {}, false, &launches};
-    if (c->sample_ev.empty()) {
-        if ((rc = plan_mover(F, S, nt, nullptr)) || (rc = plan_mover(B, *A.S, nt, &A))) return rc;
-    }
-    B.rewind();
-    if ((rc = zero_state(c, m, B.w, c->stream))) return rc;
     // normal-stress sources of the forward run: their per-target traces (source_trace)
     std::vector<int> nsrc;
     std::vector<double*> sacc;
@@ -1271,6 +1263,23 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
         nsrc.push_back((int)q);
         sacc.push_back(a);
     }
+    // the gradients and the downloads' packing: before the adjoint ring, which takes what is left
+    double* gout[3] = {};
+    for (auto& p : gout)
+        if ((rc = S.alloc(&p, slab))) return rc;
+    int64_t n3[3];
+    shape_of(g.ndim, g.order, g.physics, g.n, GPI_TAUXX, n3);
+    double* pack;
+    if ((rc = S.alloc(&pack, (size_t)(n3[0] * n3[1] * n3[2])))) return rc;
+    // the adjoint wavefield: its arrays around up to IMAGE_STEPS steps
+    AdjointRing A(c);
+    if ((rc = A.take(m, all, true))) return rc;
+    Mover B{c, m, A.st, A.ring, src2, XV2, XS2, {}, false, &launches};
+    if (c->sample_ev.empty()) {
+        if ((rc = plan_mover(F, S, nt, nullptr)) || (rc = plan_mover(B, *A.S, nt, &A))) return rc;
+    }
+    B.rewind();
+    if ((rc = zero_state(c, m, B.w, c->stream))) return rc;
     E.slab = m.slab;
     E.slots = B.ring.slots;
     E.vshift = A.inplace() ? 0 : 1;
@@ -1309,17 +1318,12 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
         }
     }
     if ((rc = finish_timing(c, smp, nt, launches))) return rc;
-    double* gout[3] = {};
-    for (auto& p : gout)
-        if ((rc = S.alloc(&p, slab))) return rc;
     elastic_gradient(m, E, gout[0], gout[1], gout[2], c->stream);
     for (size_t q = 0; q < nsrc.size(); ++q) source_correction(m, R.src.pts[nsrc[q]], sacc[q], E.nn, gout[0], gout[1], c->stream);
     HIPTRY(c, hipGetLastError());
-    int64_t n3[3];
-    shape_of(g.ndim, g.order, g.physics, g.n, GPI_TAUXX, n3);
     double* host[3] = {g_invlambda, g_invmu, g_rho};
     for (int q = 0; q < 3; ++q)
-        if ((rc = download_pitched(c, m, host[q], gout[q], n3))) return rc;
+        if ((rc = download_pitched(c, m, host[q], gout[q], n3, pack))) return rc;
     return GPI_OK;
 }
 
