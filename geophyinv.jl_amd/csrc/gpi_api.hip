@@ -175,6 +175,7 @@ int gpi_create(gpi_ctx** out, int device, uint64_t hbm_budget_bytes)
     size_t fr = 0, tot = 0;
     (void)hipMemGetInfo(&fr, &tot);
     c->budget = hbm_budget_bytes ? hbm_budget_bytes : (uint64_t)fr;
+    c->own_budget = hbm_budget_bytes != 0;
     c->keep_cap = std::min<uint64_t>((uint64_t)tot / 32, (uint64_t)8 << 30);
     *out = c;
     return GPI_OK;

@@ -151,6 +151,7 @@ struct Ctx {
     hipEvent_t ev[4] = {};
     std::vector<hipEvent_t> sample_ev;   // 4 events per sampled step
     uint64_t budget = 0, used = 0;
+    bool own_budget = false;             // `budget` was asked for (else: the free memory at creation)
     // Buffers of finished calls kept for the next ones instead of hipFree (a hipMalloc and
     // hipFree pair costs 0.1 ms for a small buffer and milliseconds for a segment of
     // wavefields): at most keep_cap bytes, freed with a model or the context, or when memory

@@ -134,9 +134,13 @@ int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void
         *p = nullptr;
         if (reuse) {
             auto k = c->kept.lower_bound(bytes);
-            if (k != c->kept.end() && k->first <= bytes + bytes / 8 + 65536) {
+            // a block up to an eighth larger, charged in full; of the same size where the caller set the
+            // budget, so that what a call needs of it does not depend on the calls before
+            const size_t slack = c->own_budget ? 0 : bytes / 8 + 65536;
+            if (k != c->kept.end() && k->first <= bytes + slack && (!c->budget || c->used + k->first <= c->budget)) {
                 *p = k->second;
                 c->kept_bytes -= k->first;
+                bytes = k->first;
                 c->kept.erase(k);
             }
         }
