@@ -187,7 +187,7 @@ struct ConvOp {
 
     int alloc(double** p, size_t n)
     {
-        hipError_t e = hipMalloc((void**)p, n * sizeof(double));
+        hipError_t e = device_malloc(c->device, (void**)p, n * sizeof(double));
         if (e != hipSuccess) return fail(c, GPI_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
         allocs.push_back(*p);
         return GPI_OK;

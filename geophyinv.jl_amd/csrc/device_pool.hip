@@ -37,7 +37,7 @@ hipError_t DevicePool::alloc(void** p, size_t bytes)
         if (carve(g, n, p)) return hipSuccess;
     const size_t size = std::max<size_t>((size_t)256 << 20, (size_t)round_up((int64_t)n, (int64_t)2 << 20));
     char* base = nullptr;
-    hipError_t e = hipMalloc((void**)&base, size);
+    hipError_t e = device_malloc(device, (void**)&base, size);
     if (e != hipSuccess) {   // give back empty segments and try once more
         (void)hipGetLastError();
         trim();

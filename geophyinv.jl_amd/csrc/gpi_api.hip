@@ -174,9 +174,10 @@ int gpi_create(gpi_ctx** out, int device, uint64_t hbm_budget_bytes)
         }
     size_t fr = 0, tot = 0;
     (void)hipMemGetInfo(&fr, &tot);
-    c->budget = hbm_budget_bytes ? hbm_budget_bytes : (uint64_t)fr;
+    c->budget = hbm_budget_bytes ? hbm_budget_bytes : (uint64_t)fr + kept_on_device(device);
     c->own_budget = hbm_budget_bytes != 0;
     c->keep_cap = std::min<uint64_t>((uint64_t)tot / 32, (uint64_t)8 << 30);
+    register_context(c);
     *out = c;
     return GPI_OK;
 }
@@ -186,6 +187,7 @@ void gpi_destroy(gpi_ctx* c)
     if (!c) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    unregister_context(c);
     for (Store* s : c->stores) free_store(c, s);
     for (Model* m : c->models) free_model(c, m);
     trim_kept(c);

@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstdint>
 #include <map>
+#include <mutex>
 #include <unordered_map>
 #include <string>
 #include <vector>
@@ -105,6 +106,7 @@ struct Store {
 // (the scheduler) allocates and frees; reserved() may be read from any thread.
 class DevicePool {
 public:
+    int device = 0;
     ~DevicePool();
     hipError_t alloc(void** p, size_t bytes);
     void free(void* p);
@@ -154,9 +156,11 @@ struct Ctx {
     bool own_budget = false;             // `budget` was asked for (else: the free memory at creation)
     // Buffers of finished calls kept for the next ones instead of hipFree (a hipMalloc and
     // hipFree pair costs 0.1 ms for a small buffer and milliseconds for a segment of
-    // wavefields): at most keep_cap bytes, freed with a model or the context, or when memory
-    // or the budget runs short.  0: nothing is kept.
+    // wavefields): at most keep_cap bytes, freed with a model or the context, when the budget runs
+    // short, or by whichever context finds the device's memory short (kept_mu: its thread frees
+    // them).  0: nothing is kept.
     uint64_t keep_cap = 0, kept_bytes = 0;
+    std::mutex kept_mu;                                // of kept, kept_bytes and block_size
     std::multimap<size_t, void*> kept;                 // size -> block
     std::unordered_map<void*, size_t> block_size;      // live and kept blocks that may be kept
     PinnedStage small;                                 // ring for the small uploads of such a context

@@ -227,7 +227,7 @@ int gpi_jobs_create(int device, const gpi_jobs_opts* opts, gpi_jobs** out)
     if (q->o.workers == 0) q->o.workers = 2;
     size_t fr = 0, tot = 0;
     (void)hipMemGetInfo(&fr, &tot);
-    q->budget = opts->hbm_budget_bytes ? opts->hbm_budget_bytes : (uint64_t)((double)fr * 0.9);
+    q->budget = opts->hbm_budget_bytes ? opts->hbm_budget_bytes : (uint64_t)((double)(fr + kept_on_device(device)) * 0.9);
     for (int k = 0; k < q->o.workers; ++k) q->workers.emplace_back([q] { q->work(); });
     *out = q;
     return GPI_OK;

@@ -794,6 +794,7 @@ int gpi_server_create(int device, const gpi_server_opts* opts, gpi_server** out)
         delete v;
         return rc;
     }
+    v->pool_dev.device = device;
     v->cc->pool = v->ac->pool = &v->pool_dev;
     v->ac->stage = &v->stage;
     v->cc->defer_free = &v->grave;
@@ -804,12 +805,12 @@ int gpi_server_create(int device, const gpi_server_opts* opts, gpi_server** out)
     v->ac->budget = 0;
     size_t fr = 0, tot = 0;
     (void)hipMemGetInfo(&fr, &tot);
-    v->budget = o.hbm_budget_bytes ? o.hbm_budget_bytes : (uint64_t)((double)fr * 0.9);
+    v->budget = o.hbm_budget_bytes ? o.hbm_budget_bytes : (uint64_t)((double)(fr + kept_on_device(device)) * 0.9);
     const size_t tb = sizeof(BatchShot2D) * v->o.max_shots + sizeof(int) * (2 * (v->o.max_shots + 1) + 1);
-    bool ok = hipMalloc((void**)&v->dtab, sizeof(BatchShot2D) * v->o.max_shots) == hipSuccess &&
-              hipMalloc((void**)&v->dfirst, sizeof(int) * (2 * (v->o.max_shots + 1) + 1)) == hipSuccess &&
-              hipMalloc((void**)&v->dmap, sizeof(uint32_t) * 2 * BATCH_MAP) == hipSuccess &&
-              hipMalloc((void**)&v->dstep, sizeof(int64_t)) == hipSuccess &&
+    bool ok = device_malloc(device, (void**)&v->dtab, sizeof(BatchShot2D) * v->o.max_shots) == hipSuccess &&
+              device_malloc(device, (void**)&v->dfirst, sizeof(int) * (2 * (v->o.max_shots + 1) + 1)) == hipSuccess &&
+              device_malloc(device, (void**)&v->dmap, sizeof(uint32_t) * 2 * BATCH_MAP) == hipSuccess &&
+              device_malloc(device, (void**)&v->dstep, sizeof(int64_t)) == hipSuccess &&
               hipStreamCreateWithFlags(&v->cap, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreateWithFlags(&v->adm_ev, hipEventDisableTiming) == hipSuccess;
     for (int k = 0; k < 2 && ok; ++k) {

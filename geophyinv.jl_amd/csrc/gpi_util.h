@@ -44,7 +44,14 @@ Model* find_model(gpi_ctx* c, uint64_t h);
 // reuse: a buffer of one call, taken from and returned to the context's kept blocks
 int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void** p, size_t bytes,
               bool reuse = false);
-void trim_kept(gpi_ctx* c);
+// frees the context's kept blocks (any thread); false: it kept none
+bool trim_kept(gpi_ctx* c);
+void register_context(gpi_ctx* c);
+void unregister_context(gpi_ctx* c);
+// bytes that the device's contexts keep, which device_malloc can have back
+uint64_t kept_on_device(int device);
+// hipMalloc; where memory is short, after every context of the device gave its kept blocks back
+hipError_t device_malloc(int device, void** p, size_t bytes);
 void free_allocs(gpi_ctx* c, std::vector<void*>& allocs, uint64_t& bytes);
 void free_model(gpi_ctx* c, Model* m);
 

@@ -112,14 +112,61 @@ Model* find_model(gpi_ctx* c, uint64_t h)
     return nullptr;
 }
 
-void trim_kept(gpi_ctx* c)
+// The contexts of the process, for their kept buffers.  Locked before a context's kept_mu; never
+// destroyed, since contexts may go after the library's statics.
+static std::mutex& g_contexts_mu = *new std::mutex;
+static std::vector<gpi_ctx*>& g_contexts = *new std::vector<gpi_ctx*>;
+
+void register_context(gpi_ctx* c)
 {
-    for (const auto& k : c->kept) {
-        c->block_size.erase(k.second);
-        (void)hipFree(k.second);
+    std::lock_guard<std::mutex> lk(g_contexts_mu);
+    g_contexts.push_back(c);
+}
+
+void unregister_context(gpi_ctx* c)
+{
+    std::lock_guard<std::mutex> lk(g_contexts_mu);
+    g_contexts.erase(std::remove(g_contexts.begin(), g_contexts.end(), c), g_contexts.end());
+}
+
+bool trim_kept(gpi_ctx* c)
+{
+    std::multimap<size_t, void*> kept;
+    {
+        std::lock_guard<std::mutex> lk(c->kept_mu);
+        kept.swap(c->kept);
+        for (const auto& k : kept) c->block_size.erase(k.second);
+        c->kept_bytes = 0;
     }
-    c->kept.clear();
-    c->kept_bytes = 0;
+    for (const auto& k : kept) (void)hipFree(k.second);   // no queued work uses them
+    return !kept.empty();
+}
+
+uint64_t kept_on_device(int device)
+{
+    std::lock_guard<std::mutex> lk(g_contexts_mu);
+    uint64_t b = 0;
+    for (gpi_ctx* c : g_contexts) {
+        if (c->device != device) continue;
+        std::lock_guard<std::mutex> lc(c->kept_mu);
+        b += c->kept_bytes;
+    }
+    return b;
+}
+
+hipError_t device_malloc(int device, void** p, size_t bytes)
+{
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    bool freed = false;
+    {
+        std::lock_guard<std::mutex> lk(g_contexts_mu);
+        for (gpi_ctx* c : g_contexts)
+            if (c->device == device && trim_kept(c)) freed = true;
+    }
+    if (!freed) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
 }
 
 int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void** p, size_t bytes, bool reuse)
@@ -132,6 +179,7 @@ int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void
     } else {
         reuse = reuse && c->keep_cap;
         *p = nullptr;
+        std::unique_lock<std::mutex> lk(c->kept_mu);
         if (reuse) {
             auto k = c->kept.lower_bound(bytes);
             // a block up to an eighth larger, charged in full; of the same size where the caller set the
@@ -145,13 +193,11 @@ int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void
             }
         }
         if (!*p) {
-            if (c->kept_bytes && c->budget && c->used + c->kept_bytes + bytes > c->budget) trim_kept(c);
-            e = hipMalloc(p, bytes);
-            if (e != hipSuccess && c->kept_bytes) {
-                (void)hipGetLastError();
-                trim_kept(c);
-                e = hipMalloc(p, bytes);
-            }
+            const bool trim = c->kept_bytes && c->budget && c->used + c->kept_bytes + bytes > c->budget;
+            lk.unlock();
+            if (trim) trim_kept(c);
+            e = device_malloc(c->device, p, bytes);
+            lk.lock();
             if (e == hipSuccess && reuse) c->block_size[*p] = bytes;
         }
     }
@@ -197,6 +243,7 @@ void free_allocs(gpi_ctx* c, std::vector<void*>& allocs, uint64_t& bytes)
     } else {
         // the caller has drained the stream; a kept block is reused on the same stream only
         for (void* p : allocs) {
+            std::unique_lock<std::mutex> lk(c->kept_mu);
             auto b = c->block_size.find(p);
             if (b != c->block_size.end() && c->kept_bytes + b->second <= c->keep_cap) {
                 c->kept.insert({b->second, p});
@@ -204,6 +251,7 @@ void free_allocs(gpi_ctx* c, std::vector<void*>& allocs, uint64_t& bytes)
                 continue;
             }
             if (b != c->block_size.end()) c->block_size.erase(b);
+            lk.unlock();
             (void)hipFree(p);
         }
     }

@@ -151,7 +151,10 @@ typedef struct gpi_timing {
 
 /* ---- context ------------------------------------------------------------------------ */
 /* No reference counterpart: the reference selects its backend at load time
- * (src/GeoPhyInv.jl:95-100).  hbm_budget_bytes = 0 means "free HBM at creation". */
+ * (src/GeoPhyInv.jl:95-100).  hbm_budget_bytes = 0 means "free HBM at creation".  A context
+ * keeps buffers of finished calls for its next ones (at most 8 GiB and 1/32 of the HBM) until one
+ * of its models is freed, its budget needs them or any context, job queue or server of the
+ * process finds the device short of memory. */
 int gpi_create(gpi_ctx** out, int device, uint64_t hbm_budget_bytes);
 void gpi_destroy(gpi_ctx* ctx);
 const char* gpi_last_error(const gpi_ctx* ctx);

@@ -557,7 +557,7 @@ hipError_t hipDeviceSynchronize()
 hipError_t hipMemGetInfo(size_t* fr, size_t* tot)
 {
     const char* e = getenv("EMU_HBM_GB");
-    const size_t total = (size_t)(e ? atof(e) : 32.0) * ((size_t)1 << 30);
+    const size_t total = (size_t)((e ? atof(e) : 32.0) * (double)((size_t)1 << 30));
     std::lock_guard<std::mutex> lk(g_mem_mu);
     *tot = total;
     *fr = total > g_live_device ? total - g_live_device : 0;

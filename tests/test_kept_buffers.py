@@ -72,3 +72,83 @@ def test_a_budget_holds_whatever_was_kept():
     for budget in ("12000000", "11800000"):
         fresh, kept = (run(BUDGET, "stores", [budget, k]).split()[-1] for k in ("fresh", "kept"))
         assert int(fresh) >= 12 and kept == fresh, (budget, fresh, kept)
+
+
+OTHERS = r"""
+from geophyinv.serve import JobServer
+def stores(ctx, p):
+    n = 0
+    try:
+        while True:
+            p.run_shot(0, save=True)
+            p._stores.pop(0)
+            n += 1
+    except _lib.GpiError as e:
+        assert e.code == -2, e
+    return n
+a = _lib.Context(0)
+pa = shot(a, 90)
+if sys.argv[1] == "kept":
+    want = pa.run_shot(0)[0]["p"].copy()
+else:
+    pa._ensure_model()
+js = JobServer(workers=1)
+queue = js.stats()["hbm_budget"]
+js.close()
+b = _lib.Context(0)
+n = stores(b, shot(b, 40))
+b.close()
+if sys.argv[1] == "kept":   # its buffers are gone, its results are not
+    assert np.array_equal(pa.run_shot(0)[0]["p"], want)
+print("stores", n, queue)
+"""
+
+
+def test_other_contexts_get_kept_buffers_back():
+    """What one idle context keeps is memory that another context and a job queue can have: as much
+    fits as if nothing were kept."""
+    env = dict(EMU_HBM_GB="0.02")
+    (n0, q0), (n1, q1) = (map(int, run(OTHERS, "stores", [k], env).split()[-2:]) for k in ("fresh", "kept"))
+    assert n0 >= 20 and n1 == n0, (n0, n1)
+    assert abs(q1 - q0) <= 256 * 50, (q0, q1)   # of some 30 buffers, which the CPU build rounds to 256 bytes
+
+
+THREADS = r"""
+import threading
+want, errors = {}, []
+def work(k, first):
+    ctx = _lib.Context(0)
+    try:
+        for nt in (60, 75, 60, 90, 75):
+            pa = shot(ctx, nt + k)
+            for _ in range(3):
+                got = pa.run_shot(0, save=True)[0]["p"].copy()
+                if first:
+                    want[nt + k] = got
+                elif not np.array_equal(got, want[nt + k]):
+                    errors.append((k, nt))
+            pa.free()
+    except Exception as e:
+        errors.append(e)
+    finally:
+        ctx.close()
+for k in range(3):
+    work(k, True)
+ts = [threading.Thread(target=work, args=(k, False)) for k in range(3)]
+[t.start() for t in ts]
+ctx, refused = _lib.Context(0, 1 << 40), 0
+big = shot(ctx, 20000)   # more than the device has: every attempt takes what the others keep
+while any(t.is_alive() for t in ts):
+    try:
+        big.run_shot(0, save=True)
+    except _lib.GpiError as e:
+        assert e.code == -2, e
+        refused += 1
+[t.join() for t in ts]
+assert not errors and refused, (errors, refused)
+print("threads agree")
+"""
+
+
+def test_contexts_on_threads_share_what_memory_there_is():
+    run(THREADS, "threads agree", env=dict(EMU_HBM_GB="0.02", EMU_THREADS="2"))
