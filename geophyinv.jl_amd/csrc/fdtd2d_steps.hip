@@ -933,6 +933,7 @@ int plan_steps_2d(gpi_ctx* c, Model& m, Scratch& S, int64_t nt, const Sources& s
 
     // ---- the second state, the coefficients and the tables, for this call alone: without room for
     // them the passes run
+    Optional spare(c);
     Scratch R(c);
     auto alt = std::make_shared<State>();
     float* co[5] = {};

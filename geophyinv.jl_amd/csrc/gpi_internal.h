@@ -153,6 +153,10 @@ struct Ctx {
     hipEvent_t ev[4] = {};
     std::vector<hipEvent_t> sample_ev;   // 4 events per sampled step
     uint64_t budget = 0, used = 0;
+    // While `optional`, what is allocated is memory that the call can do without: it may take the
+    // context up to spare_limit bytes only (0: the budget).
+    int optional = 0;
+    uint64_t spare_limit = 0;
     bool own_budget = false;             // `budget` was asked for (else: the free memory at creation)
     // Buffers of finished calls kept for the next ones instead of hipFree (a hipMalloc and
     // hipFree pair costs 0.1 ms for a small buffer and milliseconds for a segment of

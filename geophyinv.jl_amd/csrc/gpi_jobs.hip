@@ -33,7 +33,7 @@ double now_ms()
 struct Job {
     uint64_t ticket = 0;
     gpi_job j{};
-    uint64_t est = 0;
+    uint64_t est = 0, extra = 0;   // device bytes: needed, and used on top where there are any
     double t_submit = 0.0;
 };
 
@@ -83,8 +83,9 @@ uint64_t job_bytes(const gpi_job& j)
 }
 
 // Device bytes a job takes on top when they are there: the state and coefficients of the
-// several-step launches (2-D; without them the passes run) and the adjoint arrays of the
-// steps imaged together (gradients; without them every step is imaged by itself).
+// several-step launches with their sources' increments (2-D; without them the passes run) and
+// the adjoint arrays of the steps imaged together (gradients; without them every step is imaged
+// by itself).
 uint64_t job_optional_bytes(const gpi_job& j)
 {
     const gpi_grid& g = j.grid;
@@ -96,9 +97,18 @@ uint64_t job_optional_bytes(const gpi_job& j)
         const uint64_t face = std::max(ld, (uint64_t)g.n[2] + h), np = (uint64_t)std::max(g.npml, 0);
         b = (ac ? 5 : 10) * slab + (ac ? 4 : 8) * 2 * np * face * 4;
         if (j.checkpoint > 0) b *= 2;   // the adjoint wavefield's too
+        uint64_t pts = 0;
+        for (int q = 0; q < j.shot.nsrc; ++q) pts += (uint64_t)std::max(j.shot.src[q].npts, 0);
+        for (int q = 0; j.checkpoint > 0 && q < j.shot.nrec; ++q) pts += (uint64_t)std::max(j.shot.rec[q].npts, 0);
+        b += (uint64_t)j.shot.nt * 4 * pts * 4;   // four cells a point
     }
-    if (j.checkpoint > 0) b += 9 * (ac ? (d3 ? 4 : 3) : (d3 ? 9 : 5)) * slab;
-    return b;
+    if (j.checkpoint > 0) {
+        Model m;
+        m.g = g;
+        m.h = g.order - 1;
+        b += (uint64_t)(ring_steps(m) + 1) * (ac ? (d3 ? 4 : 3) : (d3 ? 9 : 5)) * slab;
+    }
+    return b * 21 / 20;
 }
 
 int run_job(gpi_ctx* c, const gpi_job& j)
@@ -169,6 +179,18 @@ struct gpi_jobs {
     int64_t submitted = 0, completed = 0, failed = 0, running = 0, fwd_done = 0, grad_done = 0;
     std::vector<double> lat, lat_f, lat_g;
 
+    // What job may use on top of its need: at most a worker's share of the budget, and what the
+    // running jobs and the next ones in the queue (as many as there are idle workers) leave.
+    // Jobs that fit together without it therefore still run together.
+    uint64_t spare(const Job& job) const
+    {
+        const uint64_t share = budget / (uint64_t)o.workers;
+        uint64_t taken = used;
+        int64_t idle = o.workers - running;
+        for (auto n = queue.begin(); n != queue.end() && idle > 0; ++n, --idle) taken += n->est;
+        return std::min({job.extra, share > job.est ? share - job.est : 0, budget > taken ? budget - taken : 0});
+    }
+
     void work()
     {
         gpi_ctx* c = nullptr;
@@ -187,10 +209,13 @@ struct gpi_jobs {
                 queue.pop_front();
                 used += job.est;
                 ++running;
+                job.extra = spare(job);
+                used += job.extra;
             }
+            if (c) c->spare_limit = job.est + job.extra;
             const int rc = crc ? crc : run_job(c, job.j);
             std::lock_guard<std::mutex> lk(mu);
-            used -= std::min(used, job.est);
+            used -= std::min(used, job.est + job.extra);
             --running;
             status[job.ticket] = rc ? rc : 0;
             if (rc) {
@@ -276,7 +301,8 @@ int gpi_jobs_submit(gpi_jobs* q, const gpi_job* job, uint64_t* ticket)
     Job x;
     x.ticket = q->next++;
     x.j = j;
-    x.est = std::min(q->budget, est + job_optional_bytes(j));
+    x.est = est;
+    x.extra = job_optional_bytes(j);
     x.t_submit = now_ms();
     q->status[x.ticket] = 1;
     q->queue.push_back(x);

@@ -528,6 +528,7 @@ int run_shot(gpi_ctx* c, Model& m, const gpi_shot* shot, Store* save)
     Ring kept;
     if (stepped && save && !ckpt) {
         std::vector<int> fields(save->field, save->field + save->nfield);
+        Optional spare(c);
         rc = alloc_ring(c, S, m, kept, fields, plan.steps + 1);
         if (rc == GPI_ENOMEM) {
             (void)hipGetLastError();
@@ -731,13 +732,9 @@ struct Mover {
     }
 };
 
-// The adjoint wavefield's arrays over up to IMAGE_STEPS steps, which one imaging launch then
+// The adjoint wavefield's arrays over up to ring_steps() steps, which one imaging launch then
 // reads together; fewer where memory is short, down to the arrays themselves (imaged between
-// the two passes of every step) where `inplace_ok`.  Where a launch takes several steps, as many
-// whole launches as twelve steps hold: with six a launch, 6 + 6 and not 6 + 2 (301 x 401 cells,
-// 700 steps, together with one strip launch for both axes: 13.1 -> 12.0 ms).
-constexpr int IMAGE_STEPS = 8;
-
+// the two passes of every step) where `inplace_ok`.
 struct AdjointRing {
     gpi_ctx* c;
     Ring ring;
@@ -763,10 +760,10 @@ struct AdjointRing {
     int take(const Model& m, const std::vector<int>& fields, bool inplace_ok)
     {
         int rc = GPI_ENOMEM;
-        const int launch = launch_steps_2d(m);
-        const int most = launch > 1 ? 12 / launch * launch : IMAGE_STEPS;
-        for (int n = most; n >= (inplace_ok ? 0 : 1) && rc == GPI_ENOMEM; n /= 2) {
+        const int least = inplace_ok ? 0 : 1;
+        for (int n = ring_steps(m); n >= least && rc == GPI_ENOMEM; n /= 2) {
             drop();
+            Optional spare(c, n > least);
             S = new Scratch(c);
             rc = alloc_ring(c, *S, m, ring, fields, n + 1);
             if (!rc) rc = alloc_state(c, m, &st, true, &ring);
@@ -786,6 +783,7 @@ int plan_mover(Mover& M, Scratch& S, int64_t nt, AdjointRing* adj)
     int rc = plan_steps_2d(c, const_cast<Model&>(M.m), S, nt, M.src, nullptr, {}, &M.plan, &M.stepped, !adj);
     if (rc || !M.stepped) return rc;
     if (adj) {
+        Optional spare(c);
         if ((rc = alloc_state(c, M.m, &adj->alt, true, &adj->ring))) {
             if (rc != GPI_ENOMEM) return rc;
             (void)hipGetLastError();
@@ -840,6 +838,15 @@ int check_shot(gpi_ctx* c, uint64_t model, const gpi_shot* shot, Model** out)
 }  // namespace
 
 namespace gpi {
+
+// Eight; where a launch takes several steps, as many whole launches as twelve steps hold: with six
+// a launch, 6 + 6 and not 6 + 2 (301 x 401 cells, 700 steps, together with one strip launch for
+// both axes: 13.1 -> 12.0 ms).
+int ring_steps(const Model& m)
+{
+    const int launch = launch_steps_2d(m);
+    return launch > 1 ? 12 / launch * launch : 8;
+}
 
 int forward_shot(gpi_ctx* c, uint64_t model, const gpi_shot* shot)
 {
@@ -1096,7 +1103,7 @@ int gpi_adjoint_checkpoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi
     shape_of(g.ndim, g.order, g.physics, g.n, GPI_P, n3);
     double* pack;   // of the downloads: before the adjoint ring, which takes what is left
     if ((rc = S.alloc(&pack, (size_t)(n3[0] * n3[1] * n3[2])))) return rc;
-    // the adjoint wavefield: p before and (for rho) v around up to IMAGE_STEPS steps
+    // the adjoint wavefield: p before and (for rho) v around the steps imaged together
     AdjointRing A(c);
     std::vector<int> kept{GPI_P};
     if (rho) kept.insert(kept.end(), vf.begin(), vf.end());
@@ -1271,7 +1278,7 @@ int gpi_adjoint_checkpoint_elastic(gpi_ctx* c, uint64_t model, uint64_t store, c
     shape_of(g.ndim, g.order, g.physics, g.n, GPI_TAUXX, n3);
     double* pack;
     if ((rc = S.alloc(&pack, (size_t)(n3[0] * n3[1] * n3[2])))) return rc;
-    // the adjoint wavefield: its arrays around up to IMAGE_STEPS steps
+    // the adjoint wavefield: its arrays around the steps imaged together
     AdjointRing A(c);
     if ((rc = A.take(m, all, true))) return rc;
     Mover B{c, m, A.st, A.ring, src2, XV2, XS2, {}, false, &launches};

@@ -44,6 +44,15 @@ Model* find_model(gpi_ctx* c, uint64_t h);
 // reuse: a buffer of one call, taken from and returned to the context's kept blocks
 int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void** p, size_t bytes,
               bool reuse = false);
+// while it lives, the context's allocations are memory that the call can do without
+struct Optional {
+    gpi_ctx* c;
+    int n;
+    explicit Optional(gpi_ctx* cc, bool on = true) : c(cc), n(on ? 1 : 0) { c->optional += n; }
+    ~Optional() { c->optional -= n; }
+    Optional(const Optional&) = delete;
+    Optional& operator=(const Optional&) = delete;
+};
 // frees the context's kept blocks (any thread); false: it kept none
 bool trim_kept(gpi_ctx* c);
 void register_context(gpi_ctx* c);
@@ -107,6 +116,8 @@ int plan_receivers(gpi_ctx* c, const Model& m, const State& st, Scratch& S, cons
 // the body of gpi_forward: one supersource on a resident model; every scratch buffer is
 // taken before the first step (from the context's arena when it has one)
 int forward_shot(gpi_ctx* c, uint64_t model, const gpi_shot* shot);
+// most adjoint steps that a gradient on this model images together
+int ring_steps(const Model& m);
 
 // model construction pieces (gpi_api.hip) and the device coefficient preparation
 // (medium.hip), shared by the C ABI and the serving scheduler

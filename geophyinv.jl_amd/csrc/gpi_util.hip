@@ -173,6 +173,8 @@ int dev_alloc(gpi_ctx* c, std::vector<void*>* owner, uint64_t* owner_bytes, void
 {
     if (c->budget && c->used + bytes > c->budget)
         return fail(c, GPI_ENOMEM, "allocation of " + std::to_string(bytes) + " bytes exceeds the context's HBM budget");
+    if (c->optional && c->spare_limit && c->used + bytes > c->spare_limit)
+        return fail(c, GPI_ENOMEM, "no spare memory for " + std::to_string(bytes) + " bytes");
     hipError_t e = hipSuccess;
     if (c->pool) {
         e = c->pool->alloc(p, bytes);
