@@ -932,8 +932,9 @@ int gpi_adjoint(gpi_ctx* c, uint64_t model, uint64_t store, const gpi_adjoint_sh
     // several steps per launch: both wavefields in rings, p of the first one forced inside the
     // launch, and one imaging launch per group of steps.  One step at a time this loop is bound by
     // its 7 launches a step (strips, four passes, imaging: about 2.5 us each); 301 x 401 cells, 700
-    // steps with the forward run: 29.9 ms, with the rings 12.0 ms
-    if (c->sample_ev.empty()) {
+    // steps with the forward run: 29.9 ms, with the rings 12.0 ms.  Orders and grids that never take
+    // several steps a launch need no rings
+    if (c->sample_ev.empty() && launch_steps_2d(m) > 0) {
         int64_t launches = 0;
         AdjointRing A1(c), A2(c);
         rc = A1.take(m, {GPI_P, GPI_VX, GPI_VZ}, false);

@@ -152,3 +152,26 @@ print("threads agree")
 
 def test_contexts_on_threads_share_what_memory_there_is():
     run(THREADS, "threads agree", env=dict(EMU_HBM_GB="0.02", EMU_THREADS="2"))
+
+
+REVERSED = r"""
+import test_time_reversal_steps as T
+held = []
+for sampling in (2, 0):   # sampled: one pass per step, no rings
+    ctx = _lib.Context(0)
+    ctx.set_pass_sampling(sampling)
+    keep, G.SeisForwExpt.free = G.SeisForwExpt.free, lambda self: None   # the model's end would free them
+    before = free_bytes()
+    T.gradient(dict(T.CASES[sys.argv[1]], nt=10), ctx)
+    held.append(before - free_bytes())
+    G.SeisForwExpt.free = keep
+print("held", *held)
+"""
+
+
+def test_time_reversal_takes_rings_only_for_several_steps():
+    """Order 8 runs pass by pass: its gradient takes (and keeps) the same buffers with and without
+    pass sampling.  Order 2 takes rings."""
+    for case, same in (("order8", True), ("odd", False)):
+        a, b = map(int, run(REVERSED, "held", [case]).split()[-2:])
+        assert (a == b) if same else (b > a), (case, a, b)
