@@ -360,10 +360,26 @@ int zero_state(gpi_ctx* c, const Model& m, const State& st, hipStream_t s)
 // Uploads up to here go through the context's pinned ring without waiting for the copy.
 static constexpr size_t SMALL_UPLOAD = (size_t)256 << 10;
 
+// The context's ring, allocated with the first upload outside the entry points that allocate
+// nothing; null: this upload waits for its copy (also where there is no pinned memory).
+static PinnedStage* small_ring(gpi_ctx* c, size_t bytes)
+{
+    if (!c->keep_cap || bytes > SMALL_UPLOAD) return nullptr;
+    if (!c->small.buf) {
+        if (c->arena) return nullptr;
+        if (hipHostMalloc((void**)&c->small.buf, 16 * SMALL_UPLOAD, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            c->small.buf = nullptr;
+            return nullptr;
+        }
+        c->small.cap = 16 * SMALL_UPLOAD;
+    }
+    return &c->small;
+}
+
 int copy_h2d(gpi_ctx* c, void* dst, const void* src, size_t bytes)
 {
-    PinnedStage* st = c->stage;
-    if (!st && c->keep_cap && bytes <= SMALL_UPLOAD) st = &c->small;
+    PinnedStage* st = c->stage ? c->stage : small_ring(c, bytes);
     if (!st) {
         HIPTRY(c, hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
         return GPI_OK;
@@ -375,7 +391,7 @@ int copy_h2d(gpi_ctx* c, void* dst, const void* src, size_t bytes)
         if (st->buf) (void)hipHostFree(st->buf);
         st->buf = nullptr;
         st->cap = st->off = 0;
-        const size_t cap = std::max<size_t>(need, st == &c->small ? 16 * SMALL_UPLOAD : (size_t)64 << 20);
+        const size_t cap = std::max<size_t>(need, (size_t)64 << 20);
         HIPTRY(c, hipHostMalloc((void**)&st->buf, cap, hipHostMallocDefault));
         st->cap = cap;
     } else if (st->off + need > st->cap) {   // wrap once every queued copy has finished
