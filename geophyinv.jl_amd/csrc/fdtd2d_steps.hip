@@ -10,14 +10,17 @@
 // carries the neighbours' samples, with two barriers per step.  The expressions and their
 // order are the passes' (fdtd2d.hip), so the results are the same bit for bit; outside an
 // update's range its coefficient is zero and outside a strip the CPML update is the
-// identity, which leaves the inner loop without branches.
+// identity, which leaves the inner loop without branches.  (The identity holds for finite
+// derivatives: where a shot has overflowed, the first step's infinities may be NaN here.  The same
+// samples are non-finite and the finite ones equal; a select per derivative that keeps the
+// infinities took 2.8 % of an elastic gradient on 251 x 333 cells and 6 % of a shot on 301^2.)
 //
 // The passes read and write 48 (acoustic) or 72 (elastic) bytes per cell and step and launch
 // twice a step, which bounds grids below about 600 cells a side by the launches (3.6 us
 // each).  Here a tile's arrays (6 in, 3 out; elastic 10 in, 5 out) move once per launch:
 // 2-D elastic 2081^2 takes 16 us a step (269 Gcell-steps/s) against 53, where the inner
-// tiles' time is half memory traffic, half arithmetic (36 vector instructions per cell and
-// step, 1.5 times the owned cells); acoustic 241^2 takes 1.4 us a step against 7.3, bound by
+// tiles' time is half memory traffic, half arithmetic (the compiled loop has 33 vector and 7
+// workgroup-memory instructions per cell and step, for 1.5 times the owned cells); acoustic 241^2 takes 1.4 us a step against 7.3, bound by
 // the latency of a launch and of the two barriers per step.
 #include "fdtd2d.h"
 #include "fdtd2d_steps.h"
@@ -689,10 +692,22 @@ int64_t frame_tiles(const Frame& f, const StepTile& t, int lead)
 // quarter of the tiles in flight) go to a launch of their own.  us per step, order 2,
 // absorbing width 20, against the passes: acoustic 260^2 1.59 / 7.2, 400^2 2.15 / 7.5,
 // 700^2 3.4 / 9, 1500^2 6.5 / 25; elastic 260^2 1.91 / 8.3, 700^2 4.8 / 13, 1500^2 10.4 / 31,
-// 2001^2 (width 40) 16.1 / 53 (8 steps there: 18.5).  Order 4: acoustic 260^2 3.4 / 7.3,
-// 497x811 (width 43) 6.5 / 9.7, 1500^2 13.3 / 25; elastic 260^2 4.3 / 8.4, 1500^2 26 / 34.  Order 6, whose halo is five
-// cells a step, gains on small grids only (260^2: 4.9 / 7.4 and 7.0 / 8.5; 400^2 lost), and
-// order 8 nowhere (1500^2 one step: 76 / 25).
+// 2001^2 (width 40) 16.1 / 53.  Order 4: acoustic 260^2 3.4 / 7.3, 497x811 (width 43) 6.5 / 9.7,
+// 1500^2 13.3 / 25; elastic 260^2 4.3 / 8.4, 1500^2 26 / 34.  Order 6, whose halo is five cells a
+// step, gains on small grids only (260^2: 4.9 / 7.4 and 7.0 / 8.5; 400^2 lost), and order 8 nowhere
+// (1500^2 one step: 76 / 25).
+// The lines between the shapes, us per step on the extended grid:
+// - order 2, 6 steps from 3 M cells, 8 below (6 / 8 steps, width 40): acoustic 1650^2 7.8 / 8.1,
+//   1760^2 8.0 / 8.2, 1900^2 8.4 / 10.0, 2081^2 9.1 / 10.6, 2400^2 11.8 / 12.1; elastic 1650^2
+//   12.3 / 13.1, 1760^2 12.5 / 13.9, 1900^2 13.7 / 16.2, 2081^2 16.4 / 18.8, 2400^2 22.7 / 22.7.
+//   Below the line the two are within 7 % (1300^2: 6.7 / 6.9 and 10.1 / 10.3); 7 steps, which the
+//   rule does not know, took 6.1 and 9.2 there and 7 to 13 % more than 6 steps from 1900^2 to 2081^2.
+// - order 2, one round of 32 x 32 tiles or of 32 x 32 around 64 x 32, and no whole grid of 64 x 32:
+//   383x483 acoustic 2.04 and elastic 2.58 against 1.86 and 2.73 in one round of 64 x 32 at 8 steps,
+//   450^2 2.09 and 2.69 against 2.42 and 3.39.
+// - order 4 acoustic, up to two rounds of 64 x 64 whole tiles at 3 steps where the frame takes more
+//   than one: 583x897 6.7 against 8.3 with the frame apart and 8.0 in one round at 2 steps,
+//   700^2 6.0 / 8.4 / 8.1; the frame apart gains at the upper end, 760x900 10.0 / 9.2 / 10.6.
 bool pick_tiles(const Model& m, StepTile* all, StepTile* inner)
 {
     constexpr int CUS = 256;

@@ -933,8 +933,8 @@ __global__ __launch_bounds__(64 * TY) void vel3d_elastic_staged(VelParams3D P, P
     }
 }
 
-// (both passes: the update reads its parameters anew each plane, fresh(): 359 against 340 us
-// a step on 190 x 201 x 210, 180 against 162 on 140 x 136 x 151, 1644 against 1598 on 360^3;
+// (both passes: the update reads its parameters anew each plane, fresh(): 340 us a step against
+// 359 without on 190 x 201 x 210, 162 against 180 on 140 x 136 x 151, 1598 against 1644 on 360^3;
 // taken there for the z-strips too, the stress pass ran 3 % slower.  Loading the x and y
 // strips' memory variables a plane ahead like the z-strips', in registers freed by a third
 // staging slot, ran 14 - 25 % slower: more loads and scalar work on every plane.)

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256) void negate_kernel(float* dst, const float* sr
 
 // Both axes' strips of consecutive steps out of a ring of a 2-D field: step blockIdx.y's values
 // in slot start + blockIdx.y, its store one strip behind the step's before.  Bound by the launch
-// (6 planes a side of each axis): one for 2 axes x 6 steps instead of one each.
+// (3 planes at each end of each axis): one for 2 axes x 6 steps instead of one each.
 struct StripRing {
     StripParams P[2];   // z, x
     const float* ring;
