@@ -307,8 +307,9 @@ __device__ __forceinline__ void run_tile(const StepParams2D& P, const TileLds& Q
         }
         const float* amp = Q.amp + (s & 1) * MAX_TILE_SOURCES;
         // columns whose values are still needed: the rest of the halo is stale already
-        const int need0 = (cxl - c0) - (P.steps - 1 - s) * H;
-        const int need1 = (cxh - c0) + (P.steps - s) * H;
+        const int halo = SR ? P.lead : cxl - c0;
+        const int need0 = halo - (P.steps - 1 - s) * H;
+        const int need1 = halo + (cxh - cxl) + (P.steps - s) * H;
         gather(false, it);
         if (lc0 + K > need0 && lc0 < need1) {
             if (PP && edge) {   // the free surface's row is written by the row below
