@@ -179,12 +179,14 @@ struct gpi_jobs {
     int64_t submitted = 0, completed = 0, failed = 0, running = 0, fwd_done = 0, grad_done = 0;
     std::vector<double> lat, lat_f, lat_g;
 
-    // What job may use on top of its need: at most a worker's share of the budget, and what the
-    // running jobs and the next ones in the queue (as many as there are idle workers) leave.
-    // Jobs that fit together without it therefore still run together.
+    // What job may use on top of its need: at most its share of the budget among as many jobs like
+    // it as the workers and the budget hold, and what the running jobs and the next ones in the
+    // queue (as many as there are idle workers) leave.  Jobs that fit together without it
+    // therefore still run together.
     uint64_t spare(const Job& job) const
     {
-        const uint64_t share = budget / (uint64_t)o.workers;
+        const uint64_t fit = std::max<uint64_t>(1, budget / std::max<uint64_t>(1, job.est));
+        const uint64_t share = budget / std::min<uint64_t>((uint64_t)o.workers, fit);
         uint64_t taken = used;
         int64_t idle = o.workers - running;
         for (auto n = queue.begin(); n != queue.end() && idle > 0; ++n, --idle) taken += n->est;

@@ -53,9 +53,9 @@ def flat(o):
     return [a for k in sorted(o) for a in ([o[k][f] for f in sorted(o[k])] if isinstance(o[k], dict) else [o[k]])]
 
 one, _, _ = serve(0, 1, 1)
-for factor in (1.0, 1.6, 8.0):
+for factor, workers in ((1.0, 2), (1.0, 3), (1.6, 2), (8.0, 2)):
     budget = int(2 * need * factor)
-    out, together, most = serve(budget, 2, 3)
+    out, together, most = serve(budget, workers, 3)
     print(sys.argv[1], need, factor, together, most, flush=True)
     assert together == 2, (factor, together)
     assert most <= budget + 256 * 400, (factor, most, budget)   # the CPU build rounds to 256 bytes
